@@ -1,0 +1,108 @@
+"""Kernel variants at the sizes where their tiling can go wrong: point sets
+around the sampler's 16 points per wavefront and its cell-map thresholds, MSI
+backgrounds whose layers and columns do not fill the scatter's 8-layer window or
+wrap onto slots of the same parity."""
+import numpy as np
+import pytest
+import torch
+
+import oracle.oracle as O
+import svox2_amd
+from svox2_amd import _C, scenes
+from tests.conftest import host_grid
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(sc, dev, dtype=torch.float32):
+    g = scenes.to_sparse_grid(sc, device=dev, dtype=dtype)
+    g.opt.sigma_thresh, g.opt.stop_thresh = 1e-8, 1e-7
+    return g
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 1000, 32768])
+@pytest.mark.parametrize("kind", ["dense", "sparse"])
+def test_sample_point_sets(gpu, kind, n):
+    """Values within 1e-5 and gradients within 1e-5 of the largest (float32
+    sums of at most a few hundred terms, 2^-24 each) of float64 sampling, with
+    and without the cell map; points outside the grid clamp to its border."""
+    gen = torch.Generator().manual_seed(n)
+    spec = scenes.BlobSpec(4, (0.2, 0.2), (20.0, 20.0))
+    sc = scenes.make_blob_grid(20, spec, gen, dense=kind == "dense")
+    grid = _grid(sc, gpu)
+    pts = torch.rand(n, 3, generator=gen) * 2.2 - 1.1
+    gd, gs = torch.randn(n, 1, generator=gen), torch.randn(n, 27, generator=gen)
+    links, dens = sc.links.numpy(), sc.density.double().float().double().requires_grad_()
+    sh = sc.sh.float().double().requires_grad_()
+    N = np.array(links.shape, np.float64)
+    f32 = np.float32
+    pg = (pts.numpy() * f32(0.5 * N[0]) + f32(0.5 * N[0] - 0.5)).astype(f32)
+    d64, s64 = O.sample_trilerp(links, dens, sh, pg)
+    torch.autograd.backward([d64, s64], [gd.double(), gs.double()])
+    for cmap in (None, False):
+        s = grid._to_cpp()
+        s.cell_map = False if cmap is False else _C.build_cell_map(s.links, grid.sh_data.size(0))
+        p = pts.to(gpu)
+        d, c = _C.sample_grid(s, p, True)
+        only, _ = _C.sample_grid(s, p, False)
+        assert torch.equal(only, d)
+        assert (d.cpu().double() - d64.detach()).abs().max() <= 1e-5 * 20
+        assert (c.cpu().double() - s64.detach()).abs().max() <= 1e-5
+        out = [torch.zeros(grid.sh_data.size(0), k, device=gpu) for k in (1, 27)]
+        _C.sample_grid_backward(s, p, gd.to(gpu), gs.to(gpu), out[0], out[1], True)
+        for got, want in zip(out, (dens.grad, sh.grad)):
+            assert (got.cpu().double() - want).abs().max() <= 1e-5 * want.abs().max().clamp_min(1)
+
+
+@pytest.mark.parametrize("n", [10, 40000, 600000])
+def test_sample_gradients_are_contiguous(gpu, n):
+    """Whatever layout the backward adds into, .grad is contiguous and equals
+    the explicit call's."""
+    gen = torch.Generator().manual_seed(3)
+    sc = scenes.make_blob_grid(96, scenes.BlobSpec(4, (0.1, 0.1), (20.0, 20.0)), gen)
+    grid = _grid(sc, gpu)
+    pts = (torch.rand(n, 3, generator=gen) * 2 - 1).to(gpu)
+    d, s = grid.sample(pts)
+    (d.sum() + s.sum()).backward()
+    want = [torch.zeros(grid.sh_data.size(0), k, device=gpu) for k in (1, 27)]
+    _C.sample_grid_backward(grid._to_cpp(), pts, torch.ones_like(d), torch.ones_like(s),
+                            want[0], want[1], True)
+    for p, w in ((grid.density_data, want[0]), (grid.sh_data, want[1])):
+        assert p.grad.is_contiguous()
+        assert (p.grad - w).abs().max() <= 1e-5 * w.abs().max()
+
+
+@pytest.mark.parametrize("reso,layers", [(4, 2), (5, 7), (7, 8), (6, 9), (9, 17), (33, 64)])
+def test_background_backward_windows(gpu, reso, layers):
+    """Background gradients of the fused step for odd and even reso (columns
+    wrap onto a slot of the same parity when reso is odd) and layer counts around
+    multiples of 8, a third of the columns empty: within 2e-5 of the largest of
+    float64 autograd; touched layers: nothing outside the trilinear cells of
+    live samples, every layer with a gradient marked."""
+    gen = torch.Generator().manual_seed(reso * 100 + layers)
+    sc = scenes.make_blob_grid(16, scenes.BlobSpec(3, (0.2, 0.2), (3.0, 3.0)), gen)
+    grid = _grid(sc, gpu)
+    links = torch.arange(2 * reso * reso, dtype=torch.int32).view(2 * reso, reso)
+    empty = torch.rand(2 * reso, reso, generator=gen) < 0.33
+    links[empty] = -1
+    links[~empty] = torch.arange(int((~empty).sum()), dtype=torch.int32)
+    rows = int((~empty).sum())
+    data = torch.randn(rows, layers, 4, generator=gen) * 0.5
+    data[..., 3] = torch.rand(rows, layers, generator=gen)
+    grid.background_nlayers, grid.background_reso = layers, reso
+    grid.background_links = links.to(gpu)
+    grid.background_data = torch.nn.Parameter(data.to(gpu))
+    o, d = scenes.sphere_rays(300, gen, radius=0.7, target=0.6)
+    gt = torch.rand(300, 3, generator=gen)
+    grid.volume_render_fused(svox2_amd.Rays(o.to(gpu), d.to(gpu)), gt.to(gpu))
+    g = host_grid(sc, links=grid.links.cpu().numpy())
+    bg = O.Background(links.numpy(), data.double().numpy())
+    data64 = data.double().requires_grad_()
+    rgb = O.render_bg_fp64(g, bg, o.numpy(), d.numpy(), O.Opts(sigma_thresh=1e-8, stop_thresh=1e-7),
+                           torch.from_numpy(g.density), torch.from_numpy(g.sh), data64)
+    ((rgb - gt.double()) ** 2).sum().div(3 * 300).backward()
+    got, want = grid.background_data.grad.cpu().double(), data64.grad
+    assert (got - want).abs().max() <= 2e-5 * want.abs().max()
+    marked = grid.sparse_background_indexer.cpu()
+    assert marked[(want.abs() > 1e-6 * want.abs().max()).any(-1)].all()
+    assert not (got[~marked] != 0).any()
