@@ -292,7 +292,8 @@ int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
  *   for batches below that threshold the forward writes every contributing
  *   sample (position, corner links, colour, transmittance) to a record
  *   stream in the workspace and the backward replays it instead of
- *   re-marching the ray (a ray whose records do not fit is re-marched);
+ *   re-marching the ray (a ray whose records do not fit is re-marched; any
+ *   bytes beyond hold more records);
  *   for batches at or above it the forward also logs where it placed the
  *   samples of each ray's first 16 chunks, and the backward evaluates those
  *   chunks from the log instead of placing them again.

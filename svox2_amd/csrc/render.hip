@@ -806,7 +806,8 @@ struct RecStream {
     // Counters, one per partition of rays (ray % parts), so that no single
     // address takes every ray's atomic: [p] overflow slots taken of opart,
     // [kRecParts + p] segment list entries of spart, [2 kRecParts + p] chunk
-    // list entries of cpart; partition p owns the p-th slice of each region.
+    // list entries of cpart; partition p owns every parts-th overflow block and
+    // the p-th slice of each list.
     uint32_t* __restrict__ next_block;
     int parts;
     int64_t opart, spart, cpart;
@@ -954,7 +955,11 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                             if (static_cast<int64_t>(nb) + kRecBlock > rs->opart) {
                                 rec_ok = false;
                             } else {
-                                const int64_t nxt = rs->overflow_base + part * rs->opart + nb;
+                                // The partitions' blocks take turns, so that
+                                // the blocks in use lie together.
+                                const int64_t nxt = rs->overflow_base +
+                                                    static_cast<int64_t>(nb) * rs->parts +
+                                                    part * kRecBlock;
                                 if (lane == 0) put_header(rs->rec, cur, 0, nxt);
                                 cur = nxt;
                                 end = nxt + kRecBlock;
@@ -1059,11 +1064,11 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
         if (lane == 0) {
             if (rec_ok) put_header(rs->rec, cur, -1, 0);
             rs->state[ray] = rec_ok ? 1 : 2;
-            for (int m = 1; m < kRecSegs; ++m)
-                if (!rec_ok || m * kRecSegChunks >= n_rec_chunks)
-                    rs->seg[ray * (kRecSegs - 1) + m - 1] = -1;
             rs->split[ray] = listed ? 1 : -1;
         }
+        const int m_end = 1 + lane;  // segments the ray does not have
+        if (m_end < kRecSegs && (!rec_ok || m_end * kRecSegChunks >= n_rec_chunks))
+            rs->seg[ray * (kRecSegs - 1) + m_end - 1] = -1;
     }
     if (LOG) {
         const int n_logged = static_cast<int>(min(n_chunks, static_cast<uint32_t>(kLogChunks)));
@@ -1605,13 +1610,13 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
                                                         RecStream rs) {
     const int lane = threadIdx.x % kGroup;
     const int64_t gid = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
-    const int64_t ngroups = static_cast<int64_t>(gridDim.x) * (kBlock / kGroup);
-    const int64_t total = rs.parts * rs.cpart;
-    for (int64_t j = gid; j < total; j += ngroups) {
-        const int64_t part = j / rs.cpart;
-        if (j - part * rs.cpart >= min(static_cast<int64_t>(rs.next_block[2 * kRecParts + part]),
-                                       rs.cpart))
-            continue;  // past the partition's entries
+    // Each partition's entries go round its share of the groups.
+    const int64_t per_part = static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) / rs.parts;
+    const int64_t part = gid % rs.parts;
+    if (gid >= per_part * rs.parts) return;
+    const int64_t entries = min(static_cast<int64_t>(rs.next_block[2 * kRecParts + part]), rs.cpart);
+    for (int64_t l = gid / rs.parts; l < entries; l += per_part) {
+        const int64_t j = part * rs.cpart + l;
         const int2 e = rs.clist[j];
         if (e.x < 0) continue;  // entries of a ray whose list did not fit
         const int64_t ray = e.x, slot = e.y;
@@ -2406,45 +2411,16 @@ SVOX2_BWD_KERNEL void k_render_backward(
     march_backward<DT, B>(g, o, r, rc, lane, st, go);
 }
 
-// Backward of the fused MSE step for the rays whose samples the forward
-// recorded (state 1): the same gradient as k_render_backward_mse, from the
-// records, in a kernel without the march code (fewer registers, more waves).
-// The ray's colour is the sum of its chunk colours (k_rec_colours) in march
-// order plus the background term, as the forward forms it; the group of item
-// < n writes it to rgb_out.  A segment m >= 1 of a split ray starts from the
-// colour composited before its first chunk.
+// One item of the replay: a ray's recorded chunks from header slot pos on, at
+// most max_chunks of them.  seg_chunk: recorded chunks before them (segments
+// m >= 1 of a split ray), or -1 from the ray's start; that item writes the
+// ray's colour.
 template <typename DT, int B>
-SVOX2_REPLAY_KERNEL void k_render_backward_replay(
-        GridView<DT> g, const float* __restrict__ dirs, int64_t n,
-        const float* __restrict__ rgb_gt, float* __restrict__ rgb_out,
-        const float* __restrict__ log_t_fwd, float beta_per_ray, float sparsity, float norm,
-        const uint32_t* __restrict__ order, GradOut go, RecStream rs) {
-    const int64_t item = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
-    const int lane = threadIdx.x % kGroup;
-    int64_t ray, pos;
-    int max_chunks = kMaxIters;
-    int seg_chunk = -1;  // recorded chunks before the segment (segments m >= 1)
-    if (item < n) {  // a ray from its start; a split ray's first segment only
-        ray = order != nullptr ? static_cast<int64_t>(order[item]) : item;
-        if (rs.state[ray] != 1) return;  // re-marched by k_render_backward_mse
-        pos = ray * rs.fixed;
-        if (rs.split[ray] >= 0) max_chunks = kRecSegChunks;
-    } else {  // a listed segment m >= 1 of a split ray
-        const int64_t e = item - n;
-        if (e >= rs.parts * rs.spart) return;
-        const int64_t part = e / rs.spart;
-        if (e - part * rs.spart >= min(static_cast<int64_t>(rs.next_block[kRecParts + part]),
-                                       rs.spart))
-            return;  // past the partition's entries
-        const int2 sm = rs.seg_list[e];
-        if (sm.x < 0) return;  // entries of a ray whose segments did not fit
-        ray = sm.x;
-        const int m = sm.y;
-        pos = rs.seg[ray * (kRecSegs - 1) + m - 1];
-        if (pos < 0) return;  // the ray ends before this segment
-        if (m < kRecSegs - 1) max_chunks = kRecSegChunks;
-        seg_chunk = m * kRecSegChunks;
-    }
+__device__ __forceinline__ void replay_item(
+        const GridView<DT>& g, const float* dirs, const float* rgb_gt, float* rgb_out,
+        const float* log_t_fwd, float beta_per_ray, float sparsity, float norm,
+        const GradOut& go, const RecStream& rs, int lane, int64_t ray, int64_t pos,
+        int max_chunks, int seg_chunk, BwdShared* sh) {
     const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
     const RayCtx<B> rc(wd);
     // The ray's colour, and the colour composited before the segment.
@@ -2470,7 +2446,7 @@ SVOX2_REPLAY_KERNEL void k_render_backward_replay(
         c3[c] += info.z;
         gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
     }
-    if (item < n && lane < 3) rgb_out[3 * ray + lane] = pick3(c3, lane);
+    if (seg_chunk < 0 && lane < 3) rgb_out[3 * ray + lane] = pick3(c3, lane);
     float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
     if (beta_per_ray > 0.f) {
         const float tin = __expf(log_t_fwd[ray]);
@@ -2478,9 +2454,53 @@ SVOX2_REPLAY_KERNEL void k_render_backward_replay(
     }
     if (seg_chunk >= 0)  // accum after the samples before the segment
         accum -= fmaf(before[0], gq[0], fmaf(before[1], gq[1], before[2] * gq[2]));
-    __shared__ BwdShared sh;
-    BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
+    BwdRay<B> st(rc, lane, gq, accum, sparsity, sh, go);
     replay_backward<DT, B>(g, rs, pos, max_chunks, lane, st, go);
+}
+
+// Backward of the fused MSE step for the rays whose samples the forward
+// recorded (state 1): the same gradient as k_render_backward_mse, from the
+// records, in a kernel without the march code (fewer registers, more waves).
+// The ray's colour is the sum of its chunk colours (k_rec_colours) in march
+// order plus the background term, as the forward forms it; the group of item
+// < n writes it to rgb_out.  A segment m >= 1 of a split ray starts from the
+// colour composited before its first chunk.
+template <typename DT, int B>
+SVOX2_REPLAY_KERNEL void k_render_backward_replay(
+        GridView<DT> g, const float* __restrict__ dirs, int64_t n,
+        const float* __restrict__ rgb_gt, float* __restrict__ rgb_out,
+        const float* __restrict__ log_t_fwd, float beta_per_ray, float sparsity, float norm,
+        const uint32_t* __restrict__ order, GradOut go, RecStream rs) {
+    const int64_t item = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
+    const int lane = threadIdx.x % kGroup;
+    __shared__ BwdShared sh;
+    if (item < n) {  // a ray from its start; a split ray's first segment only
+        const int64_t ray = order != nullptr ? static_cast<int64_t>(order[item]) : item;
+        if (rs.state[ray] != 1) return;  // re-marched by k_render_backward_mse
+        replay_item<DT, B>(g, dirs, rgb_gt, rgb_out, log_t_fwd, beta_per_ray, sparsity, norm, go,
+                           rs, lane, ray, ray * rs.fixed,
+                           rs.split[ray] >= 0 ? kRecSegChunks : kMaxIters, -1, &sh);
+        return;
+    }
+    // Listed segments m >= 1 of split rays: each partition's entries go round
+    // its share of the remaining groups.
+    const int64_t sg = item - n;
+    const int64_t per_part =
+        (static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) - n) / rs.parts;
+    const int64_t part = sg % rs.parts;
+    if (sg >= per_part * rs.parts) return;
+    const int64_t entries = min(static_cast<int64_t>(rs.next_block[kRecParts + part]), rs.spart);
+    for (int64_t l = sg / rs.parts; l < entries; l += per_part) {
+        const int2 sm = rs.seg_list[part * rs.spart + l];
+        if (sm.x < 0) continue;  // entries of a ray whose segments did not fit
+        const int64_t ray = sm.x;
+        const int m = sm.y;
+        const int64_t pos = rs.seg[ray * (kRecSegs - 1) + m - 1];
+        if (pos < 0) continue;  // the ray ends before this segment
+        replay_item<DT, B>(g, dirs, rgb_gt, rgb_out, log_t_fwd, beta_per_ray, sparsity, norm, go,
+                           rs, lane, ray, pos, m < kRecSegs - 1 ? kRecSegChunks : kMaxIters,
+                           m * kRecSegChunks, &sh);
+    }
 }
 
 // Backward of the fused MSE step: dL/drgb = (rgb - gt) * 2 / (3n) from the
@@ -2693,6 +2713,20 @@ size_t logged_workspace_bytes(int64_t n) {
     return static_cast<size_t>(order + recs + heads);
 }
 
+// Record capacity beyond the least (4096 rays of a dense 64^3 grid hold about
+// 130 contributing samples each: with the least 48 slots a ray most were marched
+// twice and re-marched by the backward, 0.43 ms a step; with room for all of
+// them 0.30 ms): a workspace of more bytes scales the
+// overflow slots and the two lists by the same factor (in 1/64).
+int64_t record_scale(size_t bytes, int64_t n) {
+    const int64_t least = static_cast<int64_t>(fused_workspace_bytes(n));
+    const int64_t per_ray = 8 * 3 + 24 * kDeferCap + kRecOverflow * kRecSlotBytes;
+    const int64_t extra = static_cast<int64_t>(bytes) - least - 4 * 256;  // alignment
+    // Header slots are int32: at most 2^31 - 1 slots.
+    const int64_t most = 64 * (INT32_MAX - n * kRecFixed) / (n * kRecOverflow);
+    return std::max<int64_t>(64, std::min<int64_t>(64 + 64 * extra / (n * per_ray), most));
+}
+
 ChunkLog chunk_log(void* ws, int64_t n) {
     char* p = static_cast<char*>(ws) + order_workspace_bytes(n);
     ChunkLog log;
@@ -2701,7 +2735,8 @@ ChunkLog chunk_log(void* ws, int64_t n) {
     return log;
 }
 
-RecStream record_stream(void* ws, int64_t n) {
+RecStream record_stream(void* ws, size_t bytes, int64_t n) {
+    const int64_t scale = record_scale(bytes, n);
     char* p = static_cast<char*>(ws) + order_workspace_bytes(n);
     RecStream rs{};
     rs.state = reinterpret_cast<int32_t*>(p);
@@ -2711,28 +2746,31 @@ RecStream record_stream(void* ws, int64_t n) {
     rs.split = reinterpret_cast<int32_t*>(p);
     p += align256(4 * n);
     rs.seg_list = reinterpret_cast<int2*>(p);
-    rs.seg_cap = seg_cap_of(n);
-    p += align256(8 * seg_cap_of(n));
+    rs.seg_cap = seg_cap_of(n) * scale / 64;
+    p += align256(8 * rs.seg_cap);
     rs.next_block = reinterpret_cast<uint32_t*>(p);
     p += align256(4 * 3 * kRecParts);
     rs.ray_info = reinterpret_cast<float4*>(p);
     p += align256(16 * n);
     rs.clist = reinterpret_cast<int2*>(p);
-    rs.clist_cap = kDeferCap * n;
-    p += align256(8 * kDeferCap * n);
+    rs.clist_cap = kDeferCap * n * scale / 64;
+    p += align256(8 * rs.clist_cap);
     rs.chunk_rgb = reinterpret_cast<float4*>(p);
-    p += align256(16 * kDeferCap * n);
+    p += align256(16 * rs.clist_cap);
     rs.rec = reinterpret_cast<float4*>(p);
     rs.fixed = kRecFixed;
     rs.overflow_base = n * kRecFixed;
-    rs.overflow_slots = n * kRecOverflow;
-    // Counter partitions: one per 1024 rays of batches of 16384 rays or more,
-    // at most kRecParts, so that each partition's share of the overflow
-    // region and lists evens out over its rays; smaller batches share one
-    // counter each (their atomics are few, and their overflow region is too
-    // small to split).
-    rs.parts = n < 16384 ? 1 : static_cast<int>(std::min<int64_t>(n / 1024, kRecParts));
-    rs.opart = rs.overflow_slots / rs.parts;
+    rs.overflow_slots = n * kRecOverflow * scale / 64;
+    // Counter partitions, at most kRecParts: one per 1024 rays of batches of
+    // 16384 rays or more, so that each partition's share of the overflow
+    // region and lists evens out over its rays; one per 64 rays where there
+    // is room for four times the least (4096 rays of a dense 64^3 grid make
+    // 25000 reservations: on one counter each, 209 us of recording
+    // forward, on 64 68 us); else smaller batches share one counter
+    // each (their overflow region is too small to split).
+    const int64_t per_part = scale >= 4 * 64 ? 64 : (n < 16384 ? n : 1024);
+    rs.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n / per_part, kRecParts)));
+    rs.opart = rs.overflow_slots / kRecBlock / rs.parts * kRecBlock;
     rs.spart = rs.seg_cap / rs.parts;
     rs.cpart = rs.clist_cap / rs.parts;
     return rs;
@@ -3495,7 +3533,7 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         log = chunk_log(workspace, n_rays);
     if (workspace != nullptr && !background && fused_records(n_rays) &&
         workspace_bytes >= fused_workspace_bytes(n_rays)) {
-        rs = record_stream(workspace, n_rays);
+        rs = record_stream(workspace, workspace_bytes, n_rays);
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kSortBlock), 0, s,
                            reinterpret_cast<uint32_t*>(rs.next_block), 3 * kRecParts);
     }
@@ -3531,7 +3569,7 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         if (w.order != nullptr) launch_cost_order(w.cost, w, n_rays, s, 1, true);
         if (rs.rec != nullptr)
             hipLaunchKernelGGL((k_render_backward_replay<DT, B>),
-                               dim3(blocks_for((n_rays + rs.seg_cap) * kGroup,
+                               dim3(blocks_for((n_rays + seg_cap_of(n_rays)) * kGroup,
                                                kBlock)),
                                dim3(kBlock), 0, s, g, dirs, n_rays, rgb_gt, rgb_out, lt, beta,
                                sparsity_loss, norm, static_cast<const uint32_t*>(w.order), go, rs);

@@ -106,3 +106,43 @@ def test_background_backward_windows(gpu, reso, layers):
     marked = grid.sparse_background_indexer.cpu()
     assert marked[(want.abs() > 1e-6 * want.abs().max()).any(-1)].all()
     assert not (got[~marked] != 0).any()
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 700, 4096])
+@pytest.mark.parametrize("factor", [1.0, 1.7, 4.0, 12.0])
+def test_fused_record_capacity(gpu, dense64, n, factor):
+    """The fused call on a dense grid with workspaces from the least to twelve
+    times it (records of all, some or few rays fit; one counter or one per 64
+    rays): colours and touched rows those of the call without a workspace,
+    gradients within 1e-5 of the largest (the order of float32 atomics)."""
+    import ctypes
+    _, o, d, gt, sc = dense64
+    grid = _grid(sc, gpu)
+    rays = svox2_amd.Rays(torch.from_numpy(o[:n]).to(gpu), torch.from_numpy(d[:n]).to(gpu))
+    gt_t = torch.from_numpy(gt[:n]).to(gpu)
+    lib = _C.load_library()
+    least = lib.svox2_volume_render_cuvol_fused_workspace_bytes(n)
+    out = []
+    for nbytes in (0, int(least * factor) // 4 * 4):
+        gd, gs, _, _ = grid._get_data_grads()
+        gd.zero_()
+        gs.zero_()
+        holder = _C.GridOutputGrads()
+        holder.grad_density_out, holder.grad_sh_out = gd, gs
+        holder.mask_out = torch.zeros(gd.size(0), dtype=torch.bool, device=gpu)
+        g = _C._grid_struct(grid._to_cpp())
+        oo, dd, clip = _C._rays(rays._to_cpp())
+        gstruct = _C._grads_struct(holder, g.rows, g.sh_data_dim)
+        rgb = torch.empty(n, 3, device=gpu)
+        ws = torch.full((max(nbytes // 4, 1),), -1, dtype=torch.int32, device=gpu)
+        st = lib.svox2_volume_render_cuvol_fused(
+            ctypes.byref(g), _C._ptr(oo), _C._ptr(dd), _C._ptr(clip), n,
+            ctypes.byref(_C._opt_struct(grid.opt._to_cpp())), _C._ptr(gt_t), 0.0, 0.0,
+            _C._ptr(rgb), None, ctypes.byref(gstruct), _C._ptr(ws) if nbytes else None, nbytes,
+            _C._stream(oo))
+        assert st == 0, lib.svox2_last_error()
+        out.append([x.clone() for x in (rgb, holder.mask_out, gd, gs)])
+    a, b = out
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    for x, y in zip(a[2:], b[2:]):
+        assert (x - y).abs().max() <= 1e-5 * x.abs().max()
