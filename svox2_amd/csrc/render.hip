@@ -1224,30 +1224,19 @@ struct BwdRay {
     }
 };
 
-// One chunk's contribution to the gradients (trace_ray_cuvol_backward,
-// render_lerp_kernel_cuvol.cu:227-383).  Lane i holds sample i of the chunk if
-// live: its position (p, l), corner links, colour + 0.5 (cs), weight, log
-// transmittance after it, world step and density.  The gradient scalars are
-// formed sample-parallel - the colour factors weight * [colour >= 0] * g and
-// the density gradient ws * (total * T_after - accum), with the running
-// `accum` as a prefix sum over the chunk - and staged as LDS records with each
-// sample's 8 trilinear weights and links in parity-slot order and the slots
-// its step leaves; then the samples are added in order into the slot
-// accumulators, one fma per corner each.
+// Adds the live samples of a chunk to the gradients.  Lane i holds sample i if
+// live: its position (p, l), corner links, colour factors gc (times the lane's
+// basis value the SH gradient), density gradient gsig, and whether it marks its
+// rows as touched (a sample that does not must be the ray's last one).  The
+// terms are staged as LDS records with each sample's 8 trilinear weights and
+// links in parity-slot order and the slots its step leaves; then the samples
+// are added in order into the slot accumulators, one fma per corner each.
 template <typename DT, int B>
-__device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradOut& go,
-                                              BwdRay<B>& st, int lane, bool live,
-                                              uint32_t live_mask, const float* p, const int* l,
-                                              const int* lk, const float* cs, float weight,
-                                              float lt_after, float ws, float sigma) {
-    float total = 0.f;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) total += fmaxf(cs[a], 0.f) * st.gq[a];
-    const float run = group_scan(live ? weight * total : 0.f);
-    const float acc_s = st.accum - run;
-    st.accum -= group_lane(run, 31);
-    float gsig = ws * (total * __expf(lt_after) - acc_s);
-    if (st.sparsity > 0.f) gsig += st.sparsity * (4.f * sigma / (1.f + 2.f * (sigma * sigma)));
+__device__ __forceinline__ void scatter_samples(const GridView<DT>& g, const GradOut& go,
+                                                BwdRay<B>& st, int lane, bool live,
+                                                uint32_t live_mask, const float* p, const int* l,
+                                                const int* lk, const float* gc, float gsig,
+                                                bool marks) {
     Scatter<B>& sc = st.sc;
     // Cell of the previous live sample: an earlier lane of this chunk, or the
     // cell the scatter is in.
@@ -1313,15 +1302,14 @@ __device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradO
             q[k | 1] = pz ? a0 : a1;
         }
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-            R.val[a] = weight * ((fmaxf(cs[a], 0.f) == cs[a]) ? 1.f : 0.f) * st.gq[a];
+        for (int a = 0; a < 3; ++a) R.val[a] = gc[a];
         R.depart = depart;
         R.val[3] = gsig;
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) R.lk[kk] = q[kk];
         // Each visit of a grid point is entered by exactly one sample: mark
         // its row there (the scatter flushes it once when the visit ends).
-        if (go.mask != nullptr) {
+        if (go.mask != nullptr && marks) {
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk)
                 if (((depart >> kk) & 1) && g.valid(q[kk])) go.mask[q[kk]] = 1;
@@ -1385,6 +1373,34 @@ __device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradO
         m &= m - 1u;
     }
     wave_lds_fence();  // records are rewritten by the next chunk
+}
+
+// One chunk's contribution to the gradients (trace_ray_cuvol_backward,
+// render_lerp_kernel_cuvol.cu:227-383).  Lane i holds sample i of the chunk if
+// live: its position (p, l), corner links, colour + 0.5 (cs), weight, log
+// transmittance after it, world step and density.  The gradient scalars are
+// formed sample-parallel: the colour factors weight * [colour >= 0] * g and
+// the density gradient ws * (total * T_after - accum), with the running
+// `accum` as a prefix sum over the chunk.
+template <typename DT, int B>
+__device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradOut& go,
+                                              BwdRay<B>& st, int lane, bool live,
+                                              uint32_t live_mask, const float* p, const int* l,
+                                              const int* lk, const float* cs, float weight,
+                                              float lt_after, float ws, float sigma) {
+    float total = 0.f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) total += fmaxf(cs[a], 0.f) * st.gq[a];
+    const float run = group_scan(live ? weight * total : 0.f);
+    const float acc_s = st.accum - run;
+    st.accum -= group_lane(run, 31);
+    float gsig = ws * (total * __expf(lt_after) - acc_s);
+    if (st.sparsity > 0.f) gsig += st.sparsity * (4.f * sigma / (1.f + 2.f * (sigma * sigma)));
+    float gc[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        gc[a] = weight * ((fmaxf(cs[a], 0.f) == cs[a]) ? 1.f : 0.f) * st.gq[a];
+    scatter_samples<DT, B>(g, go, st, lane, live, live_mask, p, l, lk, gc, gsig, true);
 }
 
 // Backward of one ray by re-marching it: every chunk is rematerialised
@@ -1848,26 +1864,22 @@ SVOX2_FWD_KERNEL void k_render_nvol(GridView<DT> g, OptView o, const float* __re
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(total, lane) + (1.f - alpha) * o.bg;
 }
 
-// Adds v * (trilinear weight of corner k at p) into column col of the rows
-// of the corners with a row.
-__device__ __forceinline__ void nvol_scatter(float* base, int64_t stride, int col, const int* lk,
-                                             const float* p, float v, int rows) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        if (static_cast<uint32_t>(lk[k]) < static_cast<uint32_t>(rows))
-            atomic_add_f32(base + lk[k] * stride + col, corner_weight(k, p) * v);
-}
-
-// nvol backward of one ray per 32-lane group.  grad_in: dL/drgb [n][3], or
-// with rgb_residual the targets (the fused MSE step: g = (color_cache -
-// grad_in) * norm).
-template <typename DT, int B>
-__global__ __launch_bounds__(kBlock) void k_render_nvol_backward(
+// nvol backward of one ray per 32-lane group.  grad_in: dL/drgb [n][3], or with
+// FUSED the targets of the MSE step (g = (colour - target) * norm): the first
+// march is then the forward, and its colour is written to rgb_out.
+//
+// The first march finds the saturating sample and with it L.  The second adds
+// both passes' terms at once, per sample ws e (total - L), through the cuvol
+// backward's register scatter.  Two marches with 8 density atomics per sample
+// and pass and 27 per sample and corner for the colours, sample by sample, after
+// a forward of its own, took 590 + 136 us for 30000 rays at 256^3; this kernel
+// 370 us.
+template <typename DT, int B, bool FUSED>
+SVOX2_BWD_KERNEL void k_render_nvol_backward(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
         const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n,
-        const float* __restrict__ grad_in, const float* __restrict__ color_cache,
-        int rgb_residual, float norm, float sparsity, GradOut go) {
-    constexpr int C = 3 * B;
+        const float* __restrict__ grad_in, float* __restrict__ rgb_out, float norm,
+        float sparsity, GradOut go) {
     const int64_t ray = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (ray >= n) return;
@@ -1876,23 +1888,10 @@ __global__ __launch_bounds__(kBlock) void k_render_nvol_backward(
     const RayCtx<B> rc(wd);
     Ray r;
     setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
-    if (r.tmin > r.tmax) return;
-    float gq[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-        gq[a] = rgb_residual ? (color_cache[3 * ray + a] - grad_in[3 * ray + a]) * norm
-                             : grad_in[3 * ray + a];
-    // This lane's SH coefficient (lane < C): its channel and basis value.
-    float basis_j = 0.f;
-#pragma unroll
-    for (int j = 0; j < B; ++j) basis_j = (lane < C && lane % B == j) ? rc.basis[j] : basis_j;
-    const int my_c = lane < C ? lane / B : 0;
-
-    // Pass 1.
-    float alpha = 0.f, last = 0.f, t_sat = r.tmax;
-    bool saturated = false;
-    {
-        float t = r.tmin;
+    float total[3] = {0.f, 0.f, 0.f}, last_rgb[3] = {o.bg, o.bg, o.bg};
+    float left = 1.f;  // 1 - opacity
+    if (r.tmin <= r.tmax) {
+        float t = r.tmin, alpha = 0.f;
         bool more = true;
         int guard = 0;
         while (more && ++guard < kMaxIters) {
@@ -1903,89 +1902,87 @@ __global__ __launch_bounds__(kBlock) void k_render_nvol_backward(
             c.weight = nvol_accumulate(lane, c.contrib, e, alpha, sat);
             c.live = c.contrib && lane <= sat;
             c.live_mask = group_ballot(c.live);
-            float cs[3] = {0.f, 0.f, 0.f};
-            if (c.live_mask != 0u) chunk_colours<DT, B, true>(g, rc, c, lane, cs, nullptr);
-            // The sample's gradient scalars (live lanes).
-            float gc[3] = {0.f, 0.f, 0.f}, tot = 0.f;
-            if (c.live) {
-                float tc[3];
+            if (c.live_mask != 0u && (FUSED || sat < 32)) {
+                float cs[3] = {0.f, 0.f, 0.f}, cacc[3] = {0.f, 0.f, 0.f}, sum[3];
+                chunk_colours<DT, B, true>(g, rc, c, lane, cs, cacc);
+                add_chunk_colour(total, cacc, sum);
+                if (sat < 32) {
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const float cl = fmaxf(cs[a], 0.f);
-                    tc[a] = cl * gq[a];
-                    gc[a] = c.weight * (cl == cs[a] ? 1.f : 0.f) * gq[a];
-                }
-                tot = (tc[0] + tc[2]) + tc[1];
-                if (lane != sat) {  // not the saturating sample: its density term
-                    float gs = c.ws * e * tot;
-                    if (sparsity > 0.f)
-                        gs += sparsity * (4.f * c.sigma / (1.f + 2.f * (c.sigma * c.sigma)));
-                    if (go.gd) nvol_scatter(go.gd, go.gds, 0, c.lk, c.p, gs, g.rows);
-                    if (go.mask) {
-#pragma unroll
-                        for (int k = 0; k < 8; ++k)
-                            if (static_cast<uint32_t>(c.lk[k]) < static_cast<uint32_t>(g.rows))
-                                go.mask[c.lk[k]] = 1;
-                    }
+                    for (int a = 0; a < 3; ++a) last_rgb[a] = fmaxf(group_bcast(cs[a], sat), 0.f);
                 }
             }
-            // SH terms, sample by sample: lane = coefficient.
-            uint32_t todo = c.live_mask;
-            while (todo != 0u) {
-                const int s = __ffs(todo) - 1;
-                todo &= todo - 1u;
-                float p[3];
-                int lk[8];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) p[a] = group_bcast(c.p[a], s);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) lk[k] = group_bcast(c.lk[k], s);
-                float v = group_bcast(gc[0], s);
-                const float g1 = group_bcast(gc[1], s), g2 = group_bcast(gc[2], s);
-                v = my_c == 0 ? v : (my_c == 1 ? g1 : g2);
-                if (lane < C && v != 0.f && go.gs)
-                    nvol_scatter(go.gs, go.gss, lane, lk, p, basis_j * v, g.rows);
-            }
-            if (sat < 32) {
-                last = group_bcast(tot, sat);
-                t_sat = group_bcast(c.t, sat);
-                saturated = true;
-                break;
-            }
+            if (sat < 32) break;
             t = c.next_t;
             more = c.more;
         }
+        left = 1.f - alpha;
     }
-    if (!saturated) last = o.bg * ((gq[0] + gq[1]) + gq[2]);
-    if (last == 0.f || go.gd == nullptr) return;
-
-    // Pass 2: every evaluated sample up to the saturating one.
-    Ray r2 = r;
-    r2.tmax = t_sat;
-    float alpha2 = 0.f;
-    float t = r2.tmin;
-    bool more = true;
+    float gq[3], tc[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (FUSED) {
+            total[a] += left * o.bg;
+            gq[a] = (total[a] - grad_in[3 * ray + a]) * norm;
+        } else {
+            gq[a] = grad_in[3 * ray + a];
+        }
+        tc[a] = last_rgb[a] * gq[a];
+    }
+    if (FUSED && lane < 3) rgb_out[3 * ray + lane] = pick3(total, lane);
+    if (r.tmin > r.tmax) return;
+    const float last = (tc[0] + tc[2]) + tc[1];
+    const bool pass2 = last != 0.f && go.gd != nullptr;
+    __shared__ BwdShared sh;
+    BwdRay<B> st(rc, lane, gq, 0.f, sparsity, &sh, go);
+    float t = r.tmin, alpha = 0.f, alpha2 = 0.f;
+    bool more = true, done2 = !pass2;
     int guard = 0;
     while (more && ++guard < kMaxIters) {
         Chunk c;
-        march_chunk(g, o, r2, lane, t, 0.f, c);
-        const bool ev = lane < c.n_eval;
-        const float e = ev ? __expf(-c.ws * c.sigma) : 1.f;
-        int sat;
-        nvol_accumulate(lane, ev, e, alpha2, sat);
-        if (ev && lane < sat) {
-            nvol_scatter(go.gd, go.gds, 0, c.lk, c.p, -c.ws * e * last, g.rows);
-            if (go.mask) {
+        march_chunk(g, o, r, lane, t, 0.f, c);
+        const float x = __expf(-c.ws * c.sigma);
+        int sat, sat2;
+        c.weight = nvol_accumulate(lane, c.contrib, c.contrib ? x : 1.f, alpha, sat);
+        c.live = c.contrib && lane <= sat;
+        c.live_mask = group_ballot(c.live);
+        // Pass 2's samples: evaluated ones up to the saturating one, until
+        // their own opacity reaches 1.
+        const bool ev = lane < c.n_eval && lane <= sat;
+        nvol_accumulate(lane, ev, ev ? x : 1.f, alpha2, sat2);
+        const bool in2 = !done2 && ev && lane < sat2;
+        done2 = done2 || sat2 < 32;
+        float cs[3] = {0.f, 0.f, 0.f};
+        if (c.live_mask != 0u) chunk_colours<DT, B, true>(g, rc, c, lane, cs, nullptr);
+        float gc[3] = {0.f, 0.f, 0.f}, gsig = 0.f;
+        const bool dens = c.live && lane != sat;
+        if (c.live) {
+            float ta[3];
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (static_cast<uint32_t>(c.lk[k]) < static_cast<uint32_t>(g.rows))
-                        go.mask[c.lk[k]] = 1;
+            for (int a = 0; a < 3; ++a) {
+                const float cl = fmaxf(cs[a], 0.f);
+                ta[a] = cl * gq[a];
+                gc[a] = c.weight * (cl == cs[a] ? 1.f : 0.f) * gq[a];
+            }
+            if (dens) {
+                gsig = c.ws * x * ((ta[0] + ta[2]) + ta[1]);
+                if (sparsity > 0.f)
+                    gsig += sparsity * (4.f * c.sigma / (1.f + 2.f * (c.sigma * c.sigma)));
             }
         }
+        if (in2) gsig -= c.ws * x * last;
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) any |= g.valid(c.lk[k]);
+        const bool add = (c.live || in2) && any;
+        const uint32_t add_mask = group_ballot(add);
+        if (add_mask != 0u)
+            scatter_samples<DT, B>(g, go, st, lane, add, add_mask, c.p, c.l, c.lk, gc, gsig,
+                                   dens || in2);
         if (sat < 32) break;
         t = c.next_t;
         more = c.more;
     }
+    st.sc.flush_all(g, go, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -3094,15 +3091,19 @@ int nvol_opt(const svox2_grid_t* grid, const float* origins, const float* dirs, 
 
 int nvol_backward(const svox2_grid_t* grid, const OptView& o, const float* origins,
                   const float* dirs, const float* ray_clip, int64_t n_rays, const float* grad_in,
-                  const float* color_cache, int rgb_residual, float norm, float sparsity,
-                  const GradOut& go, hipStream_t s) {
+                  float* rgb_out, float norm, float sparsity, const GradOut& go, hipStream_t s) {
     const unsigned blocks = blocks_for(n_rays * kGroup, kBlock);
     return dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
         using DT = std::remove_pointer_t<decltype(dtp)>;
-        hipLaunchKernelGGL((k_render_nvol_backward<DT, B>), dim3(blocks), dim3(kBlock), 0, s, g,
-                           o, origins, dirs, ray_clip, n_rays, grad_in, color_cache,
-                           rgb_residual, norm, sparsity, go);
+        if (rgb_out != nullptr)
+            hipLaunchKernelGGL((k_render_nvol_backward<DT, B, true>), dim3(blocks), dim3(kBlock),
+                               0, s, g, o, origins, dirs, ray_clip, n_rays, grad_in, rgb_out,
+                               norm, sparsity, go);
+        else
+            hipLaunchKernelGGL((k_render_nvol_backward<DT, B, false>), dim3(blocks), dim3(kBlock),
+                               0, s, g, o, origins, dirs, ray_clip, n_rays, grad_in, rgb_out,
+                               norm, sparsity, go);
     });
 }
 
@@ -3145,8 +3146,8 @@ extern "C" int svox2_volume_render_nvol_backward(const svox2_grid_t* grid, const
     if (n_rays == 0) return ok();
     SVOX2_REQUIRE(grad_out != nullptr, "grad_out is NULL");
     (void)color_cache;  // the reference's backward does not read it either
-    if ((st = nvol_backward(grid, o, origins, dirs, ray_clip, n_rays, grad_out, nullptr, 0, 1.f,
-                            0.f, go, as_stream(stream))))
+    if ((st = nvol_backward(grid, o, origins, dirs, ray_clip, n_rays, grad_out, nullptr, 1.f, 0.f,
+                            go, as_stream(stream))))
         return st;
     return check_launch("volume_render_nvol_backward");
 }
@@ -3166,10 +3167,8 @@ extern "C" int svox2_volume_render_nvol_fused(const svox2_grid_t* grid, const fl
     if ((st = check_grads(grads, grid->sh_data_dim, go))) return st;
     if (n_rays == 0) return ok();
     SVOX2_REQUIRE(rgb_gt != nullptr && rgb_out != nullptr, "rgb_gt / rgb_out are NULL");
-    if ((st = svox2_volume_render_nvol(grid, origins, dirs, ray_clip, n_rays, opt, rgb_out, stream)))
-        return st;
     const float norm = 2.f / static_cast<float>(3 * n_rays);
-    if ((st = nvol_backward(grid, o, origins, dirs, ray_clip, n_rays, rgb_gt, rgb_out, 1, norm,
+    if ((st = nvol_backward(grid, o, origins, dirs, ray_clip, n_rays, rgb_gt, rgb_out, norm,
                             sparsity_loss, go, as_stream(stream))))
         return st;
     return check_launch("volume_render_nvol_fused");
