@@ -207,23 +207,12 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Sum over each aligned group of 8 lanes, in every lane of the group, by
-// data-parallel-primitive moves (VALU, no LDS round trip): lane ^ 1 and
-// lane ^ 2 by quad permutes, then the other quad by the half-row mirror
-// (lane 7 - i), which after the first two steps holds the other quad's sum.
-// Same additions in the same order as three xor-shuffle steps 1, 2, 4.
-// Every lane of the group must be active.
+// Data-parallel-primitive move (VALU, no LDS round trip); lanes without a
+// source read 0.
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float sum8(float v) {
-    v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]: lane ^ 1
-    v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]: lane ^ 2
-    v += dpp<0x141>(v);  // row_half_mirror: lane 7 - i within 8
-    return v;
-}
-
 // Inclusive prefix sum over each 32-lane group by DPP moves: shifts by 1, 2,
 // 4 and 8 within each 16-lane row (lanes shifted in read 0), then the second
 // row of each group adds the first row's total (row broadcast of lane 15).
@@ -237,13 +226,34 @@ __device__ __forceinline__ float group_scan(float v) {
     return v;
 }
 
-// Value of lane ^ BIT (BIT = 1, 2 or 4): quad permutes for 1 and 2, a
-// bit-mode swizzle (xor mask 4 within 32 lanes) for 4.
-template <int BIT>
-__device__ __forceinline__ float xor_lanes(float v) {
-    if constexpr (BIT == 1) return dpp<0xB1>(v);
-    else if constexpr (BIT == 2) return dpp<0x4E>(v);
-    else return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x101F));
+// Steps of x(lane) = x(lane - 1) - p(lane) within each 16-lane row of the rows
+// in MASK; a row's first lane keeps its x if its p is 0.  The waits are the two
+// a DPP read needs after the vector write before it.
+#define SVOX2_CHAIN_STEP(MASK) \
+    "s_nop 1\n\tv_sub_f32_dpp %0, %0, %1 row_shr:1 row_mask:" MASK " bank_mask:0xf\n\t"
+#define SVOX2_CHAIN_5(x, p, MASK)                                                        \
+    asm volatile("s_nop 4\n\t" SVOX2_CHAIN_STEP(MASK) SVOX2_CHAIN_STEP(MASK)             \
+                     SVOX2_CHAIN_STEP(MASK) SVOX2_CHAIN_STEP(MASK) SVOX2_CHAIN_STEP(MASK) \
+                 : "+v"(x) : "v"(p))
+
+// x0 - p(0) - p(1) - ... - p(lane - 1), subtracted in that order, in lanes 0 ..
+// last of each 32-lane group (lanes above: unspecified).  Each step gives one
+// more lane its value from the lane below: one instruction, where reading lane j
+// of both groups into scalars and subtracting above it takes about ten.
+// last >= 1, the same in both groups; every lane of a group that takes part is
+// active.
+__device__ __forceinline__ float subtract_chain(float x0, float p, int last) {
+    float x = x0;
+    const float shifted = dpp<0x111>(p);  // p(lane - 1), 0 in a row's first lane
+    for (int i = 0; i < min(last, 15); i += 5) SVOX2_CHAIN_5(x, shifted, "0xf");
+    if (last >= 16) {
+        // The second row starts from the first one's end (row_bcast:15).
+        const float after = x - p;
+        x = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(after),
+                                                       0x142, 0xA, 0xF, false));
+        for (int i = 16; i < last; i += 5) SVOX2_CHAIN_5(x, shifted, "0xa");
+    }
+    return x;
 }
 
 // Lane j of this lane's 32-lane group, j the same in every lane of the
@@ -277,24 +287,6 @@ __device__ __forceinline__ int wave_last_set(bool pred) {
     const unsigned long long m = __ballot(pred);
     const uint32_t a = static_cast<uint32_t>(m), b = static_cast<uint32_t>(m >> 32);
     return max(a ? 32 - static_cast<int>(__clz(a)) : 0, b ? 32 - static_cast<int>(__clz(b)) : 0);
-}
-
-// Position (0-based) of the n-th set bit of m; m must have more than n bits set.
-__device__ __forceinline__ int nth_set_bit(uint32_t m, int n) {
-    int pos = 0;
-#pragma unroll
-    for (int w = 16; w >= 1; w >>= 1) {
-        const uint32_t lo = m & ((1u << w) - 1u);
-        const int c = __popc(lo);
-        if (n >= c) {
-            n -= c;
-            m >>= w;
-            pos += w;
-        } else {
-            m = lo;
-        }
-    }
-    return pos;
 }
 
 // Per-ray constants every lane keeps: SH basis at the view direction.
@@ -548,20 +540,12 @@ __device__ __forceinline__ void eval_chunk(const GridView<DT>& g, const OptView&
     const float pcnt = c.contrib ? c.ws * c.sigma : 0.f;
 
     // Log transmittance before this lane's sample, subtracting the earlier
-    // samples' optical depths one by one in sample order.  Only lanes up to
-    // the last contributing one subtract anything (x - 0 == x), so the replay
-    // stops there, and chunks without a contribution (empty-space crawls)
-    // skip it.
-    // The replay runs to the later of the two groups' last contributions
-    // (the other group subtracts zeros there), with a wave-uniform j.
-    float lt = log_t;
-    const int n_rep = wave_last_set(c.contrib);
-    for (int j = 0; j < n_rep; ++j) {
-        const float pj = group_lane(pcnt, j);
-        if (j < lane) lt -= pj;
-    }
-    c.lt_before = lt;
-    c.lt_after = lt - pcnt;
+    // samples' optical depths one by one in sample order, up to the later of
+    // the two groups' last contributions (x - 0 == x); chunks without one
+    // (empty-space crawls) skip it.
+    const int last_hit = wave_last_set(c.contrib) - 1;
+    c.lt_before = last_hit > 0 ? subtract_chain(log_t, pcnt, last_hit) : log_t;
+    c.lt_after = c.lt_before - pcnt;
     const uint32_t stop_mask = group_ballot(c.contrib && c.lt_after < o.log_stop);
     const int first_stop = stop_mask ? (__ffs(stop_mask) - 1) : 32;
     c.stopped = first_stop < 32;
@@ -579,7 +563,11 @@ __device__ __forceinline__ void eval_chunk(const GridView<DT>& g, const OptView&
     }
     c.n_eval = n_place;
     c.n_iter = n_place + pl.n_skips;
-    c.log_t_end = n_place > 0 ? group_bcast(c.lt_after, n_place - 1) : log_t;
+    // Past the last contribution nothing is subtracted (and the chain of the
+    // lanes there may not have been walked).
+    const uint32_t hits = group_ballot(c.contrib);
+    const float lt_last = group_bcast(c.lt_after, hits ? 31 - static_cast<int>(__clz(hits)) : 0);
+    c.log_t_end = hits ? lt_last : log_t;
     c.more = pl.more;
     c.next_t = pl.next_t;
 }
@@ -675,56 +663,6 @@ __device__ __forceinline__ uint32_t backward_cost(uint32_t work) {
     return work < static_cast<uint32_t>(kCostBins) ? work : static_cast<uint32_t>(kCostBins - 1);
 }
 
-// Colours of a chunk's live samples, grouped by cell.  Consecutive live
-// samples in the same cell form a run; they share the 8 corner rows, so
-// each row is read and projected on the SH basis once per run.  Up to four
-// runs per pass, lane = (run, corner): the lane loads its corner's row of
-// the run's cell and keeps the three projections, then for each sample of
-// the run in turn weights them trilinearly at the sample's position and sums
-// the 8 corners.  emit(pass, i, act, s, col) is called by every lane for the
-// i-th sample of each pass's runs: act says whether the lane's group has a
-// sample s at step i, col (identical in the group's 8 lanes) is its raw
-// colour.  The per-sample colour is the same float computation as a
-// per-sample gather.
-template <typename DT, int B, typename Emit>
-__device__ __forceinline__ void chunk_run_colors(const GridView<DT>& g, const RayCtx<B>& rc,
-                                                 const Chunk& c, int lane, uint32_t head_mask,
-                                                 Emit&& emit) {
-    const int n_heads = __popc(head_mask);
-    const int k = lane & 7;
-    for (int pass = 0; pass * 4 < n_heads; ++pass) {
-        const int h = pass * 4 + (lane >> 3);
-        const bool has = h < n_heads;
-        const int src = has ? nth_set_bit(head_mask, h) : 0;
-        const uint32_t later = src < 31 ? (head_mask >> (src + 1)) << (src + 1) : 0u;
-        const uint32_t below_end = later ? ((1u << (__ffs(later) - 1)) - 1u) : 0xFFFFFFFFu;
-        uint32_t run = has ? (c.live_mask & below_end & (0xFFFFFFFFu << src)) : 0u;
-        int lk = __shfl(c.lk[0], src, kGroup);
-#pragma unroll
-        for (int kk = 1; kk < 8; ++kk) {
-            const int v = __shfl(c.lk[kk], src, kGroup);
-            lk = (k == kk) ? v : lk;
-        }
-        float c0 = 0.f, c1 = 0.f, c2 = 0.f;
-        if (has && g.valid(lk)) project_row<B>(g, lk, rc.basis, c0, c1, c2);
-        for (int i = 0;; ++i) {
-            const bool act = run != 0u;
-            if (!__any(act)) break;
-            const int s = act ? __ffs(run) - 1 : 0;
-            run &= run - 1u;
-            float p[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) p[a] = __shfl(c.p[a], s, kGroup);
-            const float w = corner_weight(k, p);
-            float col[3];
-            col[0] = sum8(c0 * w);
-            col[1] = sum8(c1 * w);
-            col[2] = sum8(c2 * w);
-            emit(pass, i, act, s, col);
-        }
-    }
-}
-
 // Run heads of a chunk: live samples whose previous live sample (in lane
 // order) is not in the same cell.  Runs are formed over the live samples
 // alone, so a chunk whose live samples are compacted into lanes 0 .. n - 1
@@ -736,40 +674,95 @@ __device__ __forceinline__ uint32_t run_heads(const Chunk& c, int lane) {
     return group_ballot(c.live && !(below != 0u && prev_cell == c.base));
 }
 
-// Colours of a chunk's live samples: each live lane receives its own sample's
-// colour + 0.5 in cs (before clamping), and, if acc is given, lanes with
-// lane % 8 == 0 add weight * max(colour + 0.5, 0) of their group's samples to
-// acc (the forward's composite, summed over lanes at the end of the ray).
+// LDS of one 32-lane group for chunk_colours.
+constexpr int kColourRuns = 16;  // runs projected at a time
+struct __align__(16) ColourLds {
+    float4 at[kGroup];                 // per live sample, in order: position, weight
+    int4 links[kGroup][2];             // per run: corner links
+    float4 proj[kColourRuns][6];       // per run: 8 corners x 3 channels
+    int run[kGroup];                   // per live sample: its run
+};
+
+// Colours of a chunk's live samples.  Consecutive live samples in the same cell
+// form a run; they share the 8 corner rows, so each row is read and projected on
+// the SH basis once per run.
+// - The live samples and the runs' links go to LDS in order.
+// - lane = (run, corner), four runs per pass: the lane reads its corner's row and
+//   leaves the three projections in LDS.
+// - lane = sample: each weights its run's 8 x 3 projections trilinearly.  One
+//   pass serves up to 32 samples; with the lanes still on (run, corner), each
+//   run's samples were taken in turn and summed over the 8 corners by lane
+//   moves, about 40 instructions per sample of the longest of four runs.
+// 128x128 view of the 256^3 grid in bf16: 137 -> 94 us; 800x800 view at 512^3:
+// 1.60 -> 1.43 ms (both with the transmittance chain by lane shifts).
+// sum receives the chunk's colour, the samples' weight * max(colour + 0.5, 0)
+// added in an order that depends on their ranks alone; with TO_LANES each live
+// lane receives its own sample's colour + 0.5 in cs.  The sums per sample are
+// ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)) over its corners.
 template <typename DT, int B, bool TO_LANES>
 __device__ __forceinline__ void chunk_colours(const GridView<DT>& g, const RayCtx<B>& rc,
-                                              const Chunk& c, int lane, float* cs, float* acc) {
+                                              const Chunk& c, int lane, ColourLds* sh, float* cs,
+                                              float* sum) {
     const uint32_t heads = run_heads(c, lane);
-    const uint32_t upto = (lane == 31) ? 0xFFFFFFFFu : ((2u << lane) - 1u);
-    const uint32_t my_heads = heads & upto;
-    // This lane's run (head index) and its place in the run.
-    const int my_run = __popc(my_heads) - 1;
-    const int head_pos = my_heads ? 31 - __clz(my_heads) : 0;
-    const int my_idx = __popc(c.live_mask & ((1u << lane) - 1u) & (0xFFFFFFFFu << head_pos));
-    chunk_run_colors<DT, B>(
-        g, rc, c, lane, heads, [&](int pass, int i, bool act, int s, const float* col) {
-            if (acc != nullptr) {
-                const float w = __shfl(c.weight, s, kGroup);
-                if (act && (lane & 7) == 0) {
+    const uint32_t below = (1u << lane) - 1u;
+    const int rank = __popc(c.live_mask & below);
+    if (c.live) {
+        const bool head = ((heads >> lane) & 1u) != 0;
+        const int my_run = __popc(heads & below) - (head ? 0 : 1);
+        sh->at[rank] = make_float4(c.p[0], c.p[1], c.p[2], c.weight);
+        sh->run[rank] = my_run;
+        if (head) {
+            sh->links[my_run][0] = make_int4(c.lk[0], c.lk[1], c.lk[2], c.lk[3]);
+            sh->links[my_run][1] = make_int4(c.lk[4], c.lk[5], c.lk[6], c.lk[7]);
+        }
+    }
+    wave_lds_fence();
+    const int n_runs = __popc(heads);
+    const bool has = lane < __popc(c.live_mask);
+    const float4 q = has ? sh->at[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const int run = has ? sh->run[lane] : -1;
+    const float p[3] = {q.x, q.y, q.z};
+    float col[3] = {0.f, 0.f, 0.f};
+    const int k = lane & 7;
+    for (int base = 0; base < n_runs; base += kColourRuns) {
+        const int end = min(n_runs, base + kColourRuns);
+        for (int r = base + (lane >> 3); r < end; r += 4) {
+            const int lk = reinterpret_cast<const int*>(sh->links[r])[k];
+            float c0 = 0.f, c1 = 0.f, c2 = 0.f;
+            if (g.valid(lk)) project_row<B>(g, lk, rc.basis, c0, c1, c2);
+            float* out = reinterpret_cast<float*>(sh->proj[r - base]) + 3 * k;
+            out[0] = c0;
+            out[1] = c1;
+            out[2] = c2;
+        }
+        wave_lds_fence();
+        if (run >= base && run < end) {
+            const float4* v4 = sh->proj[run - base];
+            float v[24];
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) acc[a] += w * fmaxf(col[a] + 0.5f, 0.f);
-                }
+            for (int i = 0; i < 6; ++i) {
+                const float4 x = v4[i];
+                v[4 * i] = x.x;
+                v[4 * i + 1] = x.y;
+                v[4 * i + 2] = x.z;
+                v[4 * i + 3] = x.w;
             }
-            if (TO_LANES) {
-                const int grp = my_run - 4 * pass;
-                const bool mine = c.live && grp >= 0 && grp < 4 && my_idx == i;
-                const int from = mine ? 8 * grp : 0;
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const float v = __shfl(col[a], from, kGroup);
-                    cs[a] = mine ? v + 0.5f : cs[a];
-                }
+            for (int a = 0; a < 3; ++a) {
+                float t[8];
+#pragma unroll
+                for (int kk = 0; kk < 8; ++kk) t[kk] = v[3 * kk + a] * corner_weight(kk, p);
+                col[a] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
             }
-        });
+        }
+        wave_lds_fence();  // the next runs' projections, or the caller, take the space
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float shown = col[a] + 0.5f;
+        sum[a] = group_lane(group_scan(has ? q.w * fmaxf(shown, 0.f) : 0.f), 31);
+        if (TO_LANES) cs[a] = __shfl(shown, c.live ? rank : 0, kGroup);
+    }
 }
 
 // Chunk log of the fused call: the forward writes the placement of each of a
@@ -847,22 +840,6 @@ __device__ __forceinline__ void put_header(float4* rec, int64_t slot, int n, int
                                 0.f);
 }
 
-// Adds a chunk's colour to the ray's: the run groups' partial sums (lanes 0,
-// 8, 16 and 24 of cacc) reduced across the group as (a0 + a8) + (a16 + a24),
-// lane ^ 8 by a row rotation and lane ^ 16 by a bit-mode swizzle (no LDS
-// addresses), then added to total in march order (every lane of the group
-// gets the same sums).
-__device__ __forceinline__ void add_chunk_colour(float* total, const float* cacc, float* sum) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        float v = cacc[a];
-        v += dpp<0x128>(v);  // row_ror:8 - lane ^ 8 within each 16-lane row
-        v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));  // lane ^ 16
-        sum[a] = group_lane(v, 0);
-        total[a] += sum[a];
-    }
-}
-
 // Forward march of one ray.  out[3] = composited colour (all lanes),
 // returns the final log transmittance.  A chunk's colour sums its live
 // samples' weighted colours (per run group, then across the group); the ray's
@@ -879,7 +856,7 @@ template <typename DT, int B, bool STATS, bool RECORD = false, bool LOG = false,
 __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptView& o,
                                                const Ray& r, const RayCtx<B>& rc, int lane,
                                                float* out, int32_t* stats,
-                                               uint32_t* cost = nullptr,
+                                               ColourLds* colour_lds, uint32_t* cost = nullptr,
                                                const RecStream* rs = nullptr,
                                                int64_t ray = 0,
                                                const ChunkLog* log = nullptr,
@@ -940,9 +917,10 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                                            n_rec_chunks / kRecSegChunks < kRecSegs;
                     float cs[3] = {0.f, 0.f, 0.f};
                     if (!defer) {
-                        float cacc[3] = {0.f, 0.f, 0.f}, sum[3];
-                        chunk_colours<DT, B, RECORD>(g, rc, c, lane, cs, cacc);
-                        add_chunk_colour(total, cacc, sum);
+                        float sum[3];
+                        chunk_colours<DT, B, RECORD>(g, rc, c, lane, colour_lds, cs, sum);
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) total[a] += sum[a];
                     }
                     if (RECORD && rec_ok) {
                         // Header + n_live records; keep one slot for a jump/end header.
@@ -1121,10 +1099,15 @@ struct __align__(16) SampleRec {
     int pad[3];
 };
 
-// LDS of one backward workgroup: the sample records of its rays.
+// LDS of one backward workgroup: per ray the sample records, or in the same
+// place, before they are written, the chunk's colours in the making.
 struct BwdShared {
-    SampleRec rec[kBlock];
+    union {
+        SampleRec rec[kGroup];
+        ColourLds colour;
+    } ray[kBlock / kGroup];
 };
+static_assert(std::is_trivially_default_constructible<BwdShared>::value, "used as LDS");
 
 // Gradient scatter state of one ray.  Lane L of the 32-lane group owns one
 // gradient column of a row: SH channel L (c = L / B, j = L % B) for L < C,
@@ -1205,11 +1188,12 @@ struct BwdRay {
     float sparsity;
     int my_q;        // quantity of this lane's column: c for SH lanes, 3 otherwise
     SampleRec* rec;  // this group's LDS records
+    ColourLds* colour;
     Scatter<B> sc;
 
     __device__ __forceinline__ BwdRay(const RayCtx<B>& rc, int lane, const float* g3, float acc0,
                                       float sp, BwdShared* sh, const GradOut& go) {
-        const int gbase = threadIdx.x & ~(kGroup - 1);
+        const int group = threadIdx.x / kGroup;
 #pragma unroll
         for (int a = 0; a < 3; ++a) gq[a] = g3[a];
         accum = acc0;
@@ -1219,7 +1203,8 @@ struct BwdRay {
 #pragma unroll
         for (int j = 0; j < B; ++j) basis_j = (lane < C && lane % B == j) ? rc.basis[j] : basis_j;
         my_q = lane < C ? lane / B : 3;
-        rec = sh->rec + gbase;
+        rec = sh->ray[group].rec;
+        colour = &sh->ray[group].colour;
         sc.init(go, lane, basis_j);
     }
 };
@@ -1482,8 +1467,8 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
             march_chunk(g, o, r, lane, t, log_t, c);
         }
         if (c.live_mask != 0u) {
-            float cs[3] = {0.f, 0.f, 0.f};
-            chunk_colours<DT, B, true>(g, rc, c, lane, cs, nullptr);
+            float cs[3] = {0.f, 0.f, 0.f}, sum[3];
+            chunk_colours<DT, B, true>(g, rc, c, lane, st.colour, cs, sum);
             scatter_chunk<DT, B>(g, go, st, lane, c.live, c.live_mask, c.p, c.l, c.lk, cs,
                                  c.weight, c.lt_after, c.ws, c.sigma);
         }
@@ -1604,8 +1589,9 @@ SVOX2_REC_KERNEL void k_render_rays_rec(
     uint32_t cost = 0;
     // LDS staging of this group's recorded chunk header slots.
     __shared__ int32_t slot_lds[(kBlock / kGroup) * kDeferChunks];
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, false, true, false, true>(
-        g, o, r, rc, lane, out, nullptr, cost_out != nullptr ? &cost : nullptr, &rs, ray,
+        g, o, r, rc, lane, out, nullptr, colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray,
         nullptr, nullptr, slot_lds + (threadIdx.x / kGroup) * kDeferChunks);
     // A ray whose chunks were listed gets its colour from k_rec_colours.
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
@@ -1626,6 +1612,7 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
                                                         RecStream rs) {
     const int lane = threadIdx.x % kGroup;
     const int64_t gid = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
     // Each partition's entries go round its share of the groups.
     const int64_t per_part = static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) / rs.parts;
     const int64_t part = gid % rs.parts;
@@ -1665,9 +1652,8 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
         }
         const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
         const RayCtx<B> rc(wd);
-        float cs[3] = {0.f, 0.f, 0.f}, cacc[3] = {0.f, 0.f, 0.f}, sum[3], unused[3] = {0.f, 0.f, 0.f};
-        chunk_colours<DT, B, true>(g, rc, c, lane, cs, cacc);
-        add_chunk_colour(unused, cacc, sum);
+        float cs[3] = {0.f, 0.f, 0.f}, sum[3];
+        chunk_colours<DT, B, true>(g, rc, c, lane, colour_lds + threadIdx.x / kGroup, cs, sum);
         if (c.live) {
             float* q4 = reinterpret_cast<float*>(q + 4 * n);
             q4[0] = cs[0];
@@ -1698,9 +1684,10 @@ SVOX2_FWD_KERNEL void k_render_rays(
     uint32_t cost = 0;
     // LDS staging of this group's chunk log (used when LOG).
     __shared__ float log_lds[LOG ? (kBlock / kGroup) * kLogChunks * kLogWords : 1];
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, STATS, false, LOG>(
         g, o, r, rc, lane, out, STATS ? stats + 4 * ray : nullptr,
-        cost_out != nullptr ? &cost : nullptr, &rs, ray, &log,
+        colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray, &log,
         log_lds + (threadIdx.x / kGroup) * kLogChunks * kLogWords);
     if (!STATS) {
         if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
@@ -1838,6 +1825,7 @@ SVOX2_FWD_KERNEL void k_render_nvol(GridView<DT> g, OptView o, const float* __re
     const RayCtx<B> rc(wd);
     Ray r;
     setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
     float alpha = 0.f, total[3] = {0.f, 0.f, 0.f};
     if (r.tmin <= r.tmax) {
         float t = r.tmin;
@@ -1852,9 +1840,11 @@ SVOX2_FWD_KERNEL void k_render_nvol(GridView<DT> g, OptView o, const float* __re
             c.live = c.contrib && lane <= sat;
             c.live_mask = group_ballot(c.live);
             if (c.live_mask != 0u) {
-                float cs[3], cacc[3] = {0.f, 0.f, 0.f}, sum[3];
-                chunk_colours<DT, B, false>(g, rc, c, lane, cs, cacc);
-                add_chunk_colour(total, cacc, sum);
+                float cs[3], sum[3];
+                chunk_colours<DT, B, false>(g, rc, c, lane, colour_lds + threadIdx.x / kGroup, cs,
+                                            sum);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) total[a] += sum[a];
             }
             if (sat < 32) break;
             t = c.next_t;
@@ -1889,6 +1879,7 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
     Ray r;
     setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
     float total[3] = {0.f, 0.f, 0.f}, last_rgb[3] = {o.bg, o.bg, o.bg};
+    __shared__ BwdShared sh;
     float left = 1.f;  // 1 - opacity
     if (r.tmin <= r.tmax) {
         float t = r.tmin, alpha = 0.f;
@@ -1903,9 +1894,11 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
             c.live = c.contrib && lane <= sat;
             c.live_mask = group_ballot(c.live);
             if (c.live_mask != 0u && (FUSED || sat < 32)) {
-                float cs[3] = {0.f, 0.f, 0.f}, cacc[3] = {0.f, 0.f, 0.f}, sum[3];
-                chunk_colours<DT, B, true>(g, rc, c, lane, cs, cacc);
-                add_chunk_colour(total, cacc, sum);
+                float cs[3] = {0.f, 0.f, 0.f}, sum[3];
+                chunk_colours<DT, B, true>(g, rc, c, lane, &sh.ray[threadIdx.x / kGroup].colour,
+                                           cs, sum);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) total[a] += sum[a];
                 if (sat < 32) {
 #pragma unroll
                     for (int a = 0; a < 3; ++a) last_rgb[a] = fmaxf(group_bcast(cs[a], sat), 0.f);
@@ -1932,7 +1925,6 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
     if (r.tmin > r.tmax) return;
     const float last = (tc[0] + tc[2]) + tc[1];
     const bool pass2 = last != 0.f && go.gd != nullptr;
-    __shared__ BwdShared sh;
     BwdRay<B> st(rc, lane, gq, 0.f, sparsity, &sh, go);
     float t = r.tmin, alpha = 0.f, alpha2 = 0.f;
     bool more = true, done2 = !pass2;
@@ -1951,8 +1943,8 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
         nvol_accumulate(lane, ev, ev ? x : 1.f, alpha2, sat2);
         const bool in2 = !done2 && ev && lane < sat2;
         done2 = done2 || sat2 < 32;
-        float cs[3] = {0.f, 0.f, 0.f};
-        if (c.live_mask != 0u) chunk_colours<DT, B, true>(g, rc, c, lane, cs, nullptr);
+        float cs[3] = {0.f, 0.f, 0.f}, sum[3];
+        if (c.live_mask != 0u) chunk_colours<DT, B, true>(g, rc, c, lane, st.colour, cs, sum);
         float gc[3] = {0.f, 0.f, 0.f}, gsig = 0.f;
         const bool dens = c.live && lane != sat;
         if (c.live) {
@@ -2348,7 +2340,9 @@ SVOX2_FWD_KERNEL void k_render_image(
     Ray r;
     setup_ray(g, o, wo, wd, nullptr, r);
     float out[3];
-    const float log_t = march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr);
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
+    const float log_t = march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr,
+                                                    colour_lds + threadIdx.x / kGroup);
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
     if (log_t_out != nullptr && lane == 0) log_t_out[ray] = log_t;
 }
@@ -2381,7 +2375,9 @@ SVOX2_FWD_KERNEL void k_render_tiles(const svox2_grid_t* __restrict__ grids, int
     Ray r;
     setup_ray(g, o, wo, wd, nullptr, r);
     float out[3];
-    march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr);
+    __shared__ ColourLds colour_lds[kBlock / kGroup];
+    march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr,
+                                colour_lds + threadIdx.x / kGroup);
     if (lane < 3) tile.rgb_out[3 * pixel + lane] = pick3(out, lane);
 }
 
