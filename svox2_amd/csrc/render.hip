@@ -387,23 +387,37 @@ struct Placement {
     int my_skips = 0;  // skips before this lane's sample
 };
 
+// Where a march begins: at t, on lane `lane` of its first chunk, after `skips`
+// skips in it.  Lanes below stand for samples that read no row.
+struct MarchStart {
+    float t;
+    int lane = 0;
+    int skips = 0;
+};
+
 template <typename DT>
 __device__ __forceinline__ void place_chunk(const GridView<DT>& g, const OptView& o,
-                                            const Ray& r, int lane, float t0, Chunk& c,
-                                            Placement& pl) {
+                                            const Ray& r, int lane, const MarchStart& from,
+                                            Chunk& c, Placement& pl) {
     // Place the samples.  Each round gives the lanes from seg_lane on
     // the steps of the segment starting at seg_t, reads their cells' skip
     // levels and finds the segment's end.
-    int seg_lane = 0;      // first lane of the current segment
-    float seg_t = t0;      // t of its first sample
-    int n_skips = 0;       // skips before the current segment
-    int my_skips = 0;      // skips before this lane's sample
-    bool occupied = true;  // the cell may have a corner link that addresses a row
-    float ti = t0;
+    int seg_lane = from.lane;  // first lane of the current segment
+    float seg_t = from.t;      // t of its first sample
+    int n_skips = 0;           // skips before the current segment
+    int my_skips = 0;          // skips before this lane's sample
+    bool occupied = lane >= from.lane;  // the cell may have a corner link that addresses a row
+    float ti = from.t;
+    c.base = 0;  // lanes below the start's
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        c.p[a] = 0.f;
+        c.l[a] = 0;
+    }
     int n_place;           // evaluated lanes 0 .. n_place - 1
     bool more;
     float next_t = 0.f;
-    for (int seg = 1;; ++seg) {
+    for (int seg = 1 + from.skips;; ++seg) {
         const bool mine = lane >= seg_lane;
         if (mine) {
             // t of the k-th step of the segment, as the sequential float
@@ -574,10 +588,10 @@ __device__ __forceinline__ void eval_chunk(const GridView<DT>& g, const OptView&
 
 template <typename DT>
 __device__ __forceinline__ void march_chunk(const GridView<DT>& g, const OptView& o,
-                                            const Ray& r, int lane, float t0, float log_t,
-                                            Chunk& c) {
+                                            const Ray& r, int lane, const MarchStart& from,
+                                            float log_t, Chunk& c) {
     Placement pl;
-    place_chunk(g, o, r, lane, t0, c, pl);
+    place_chunk(g, o, r, lane, from, c, pl);
     eval_chunk(g, o, r, lane, log_t, pl, c);
 }
 
@@ -854,7 +868,8 @@ __device__ __forceinline__ void put_header(float4* rec, int64_t slot, int n, int
 template <typename DT, int B, bool STATS, bool RECORD = false, bool LOG = false,
           bool DEFER = false>
 __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptView& o,
-                                               const Ray& r, const RayCtx<B>& rc, int lane,
+                                               const Ray& r, const MarchStart& start,
+                                               const RayCtx<B>& rc, int lane,
                                                float* out, int32_t* stats,
                                                ColourLds* colour_lds, uint32_t* cost = nullptr,
                                                const RecStream* rs = nullptr,
@@ -883,13 +898,13 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
             n_chunks = n_live_all = n_live_chunks = 0;
         }
         log_t = 0.f;
-        if (r.tmin <= r.tmax) {
-            float t = r.tmin;
+        if (start.t <= r.tmax) {
+            MarchStart at = start;
             int guard = 0;
             bool more = true;
             while (more && ++guard < kMaxIters) {
                 Chunk c;
-                march_chunk(g, o, r, lane, t, log_t, c);
+                march_chunk(g, o, r, lane, at, log_t, c);
                 const int n_live = __popc(c.live_mask);
                 if (LOG && n_chunks < static_cast<uint32_t>(kLogChunks)) {
                     // Staged in LDS and written out when the ray ends: global
@@ -979,7 +994,7 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                     }
                 }
                 log_t = c.log_t_end;
-                t = c.next_t;
+                at = MarchStart{c.next_t};
                 more = c.more;
                 if (DEFER && defer && !rec_ok) break;  // march again, colours here
             }
@@ -1393,10 +1408,10 @@ __device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradO
 template <typename DT, int B, bool PREFETCH = true>
 __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptView& o,
                                                const Ray& r, const RayCtx<B>& rc, int lane,
-                                               BwdRay<B>& st, const GradOut& go,
+                                               BwdRay<B>& st, const GradOut& go, float begin,
                                                ChunkLog log_v = ChunkLog{},
                                                int64_t ray = 0) {
-    if (r.tmin > r.tmax) return;
+    if (!(begin <= r.tmax)) return;
     // Chunks the forward logged are evaluated from their placement.
     int n_logged = 0;
     bool log_more = false;
@@ -1406,6 +1421,7 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
         n_logged = min(h.x, kLogChunks);
         log_more = h.y != 0;
         log_next_t = __int_as_float(h.z);
+        if (n_logged == 0) return;  // the forward met no sample that can count
     }
     // With PREFETCH the next logged chunk's placement is read, and its corner
     // links requested, while the current chunk is evaluated, so a logged
@@ -1424,7 +1440,7 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
         int nl[3];
         load_corner_links(g, lane, sample_cell(g, r, nt, np, nl), nmask, nlk);
     }
-    float t = r.tmin;
+    float t = begin;
     float log_t = 0.f;
     int guard = 0;
     bool more = true;
@@ -1464,7 +1480,7 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
                 load_corner_links(g, lane, sample_cell(g, r, nt, np, nl), nmask, nlk);
             }
         } else {
-            march_chunk(g, o, r, lane, t, log_t, c);
+            march_chunk(g, o, r, lane, MarchStart{t}, log_t, c);
         }
         if (c.live_mask != 0u) {
             float cs[3] = {0.f, 0.f, 0.f}, sum[3];
@@ -1591,7 +1607,7 @@ SVOX2_REC_KERNEL void k_render_rays_rec(
     __shared__ int32_t slot_lds[(kBlock / kGroup) * kDeferChunks];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, false, true, false, true>(
-        g, o, r, rc, lane, out, nullptr, colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray,
+        g, o, r, MarchStart{r.tmin}, rc, lane, out, nullptr, colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray,
         nullptr, nullptr, slot_lds + (threadIdx.x / kGroup) * kDeferChunks);
     // A ray whose chunks were listed gets its colour from k_rec_colours.
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
@@ -1664,13 +1680,99 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
     }
 }
 
+// Lane-per-ray search for each ray's first sample whose cell may have rows,
+// for launches of kHeadRays rays or more on a grid with a cell map.  The steps
+// and skips are those of the march (a skip or a single step per iteration), so
+// the t found is the march's own; with it go its place in its chunk (lane and
+// skips), so that chunks, and with them every sum, stay as they are without the
+// search.  Most camera rays meet no row at all (86 % of an 800x800 view of the
+// 512^3 blob grid): a lane finds that in about 23 cell-map reads, where half a
+// wavefront takes a few packed rounds.  The result goes where the ray's own
+// result will be written: words = 3, (t, lane | skips << 8, -) into the colour;
+// words = 1, t alone into the depth; infinity if there is no such sample.
+// key (may be NULL): the ray's order key, its length from there on.
+//
+// 800x800 view at 512^3: the march 1434 -> 1090 us, this kernel 90 us; 200003
+// rays in bf16: 675 -> 440 and 70 us.  Walked to the end, grazing rays hold it
+// for 616 us; at most 48, 64 and 128 steps give 1205, 1179 and 1203 us in all.
+constexpr int kHeadBlock = 256;
+constexpr int kHeadSteps = 64;
+constexpr int kHeadLanes = 4;
+
+template <bool IMAGE>
+__global__ __launch_bounds__(kHeadBlock) void k_march_start(
+        GridView<float> g, OptView o, svox2_camera_t cam, const float* __restrict__ origins,
+        const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n, int words,
+        float* __restrict__ out, float bins_per_voxel, uint32_t* __restrict__ key,
+        uint32_t* __restrict__ clear) {
+    if (key != nullptr && blockIdx.x == 0)  // both histograms of the ordering workspace
+        for (int b = threadIdx.x; b < 2 * kCostBins; b += kHeadBlock) clear[b] = 0u;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kHeadBlock + threadIdx.x;
+    if (i >= n) return;
+    float wo[3], wd[3];
+    if (IMAGE) {
+        camera_ray(cam, static_cast<int>(i % cam.width), static_cast<int>(i / cam.width), wd, wo);
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            wo[a] = origins[3 * i + a];
+            wd[a] = dirs[3 * i + a];
+        }
+    }
+    Ray r;
+    setup_ray(g, o, wo, wd, clip ? clip + 2 * i : nullptr, r);
+    MarchStart at{r.tmin};
+    // The wavefront walks on while enough of its lanes do, kHeadSteps at most;
+    // the rest is left to the march, which may begin anywhere on the walk (a ray
+    // grazing a surface for hundreds of steps would hold 63 others up).
+    bool more = at.t <= r.tmax;
+    for (int k = 0; k < kHeadSteps && __popcll(__ballot(more)) >= kHeadLanes; ++k) {
+        if (!more) continue;
+        float p[3];
+        int l[3];
+        const int base = sample_cell(g, r, at.t, p, l);
+        const uint32_t info =
+            g.cmap[(l[0] >> 1) * g.mstride_x + (l[1] >> 1) * g.mstride_y + (l[2] >> 1)];
+        int level = static_cast<int>(info & 0xFFu);
+        if (level == 255) {
+            const int l0 = g.links[base];
+            level = l0 < -1 ? -l0 - 1 : 0;
+        }
+        const float skip = level > 0 ? skip_dist(-1 - level, l, p, r) : 0.f;
+        if (skip >= o.step) {
+            at.t += ceilf(skip / o.step) * o.step;
+            if (++at.skips == kMaxSegments) at.lane = at.skips = 0;  // the chunk ends
+        } else if ((info >> (8 + ((l[0] & 1) << 2) + ((l[1] & 1) << 1) + (l[2] & 1))) & 1u) {
+            more = false;
+        } else {
+            at.t += o.step;
+            if (++at.lane == kGroup) at.lane = at.skips = 0;
+        }
+        more = more && at.t <= r.tmax;
+    }
+    const bool found = at.t <= r.tmax;
+    out[words * i] = found ? at.t : INFINITY;
+    if (words > 1) out[words * i + 1] = __int_as_float(at.lane | (at.skips << 8));
+    if (key != nullptr)
+        key[i] = found ? static_cast<uint32_t>(fminf((r.tmax - at.t) * bins_per_voxel + 1.f,
+                                                     static_cast<float>(kCostBins - 1)))
+                       : 0u;
+}
+
+// Where a ray's march begins: what k_march_start left at found, or tmin.
+__device__ __forceinline__ MarchStart start_of(const Ray& r, const float* found) {
+    if (found == nullptr) return MarchStart{r.tmin};
+    const int place = __float_as_int(found[1]);
+    return MarchStart{found[0], place & 0xFF, place >> 8};
+}
+
 template <typename DT, int B, bool STATS, bool LOG = false>
 SVOX2_FWD_KERNEL void k_render_rays(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
         const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n,
         float* __restrict__ rgb_out, float* __restrict__ log_t_out,
         int32_t* __restrict__ stats, uint32_t* __restrict__ cost_out, RecStream rs,
-        const uint32_t* __restrict__ order, ChunkLog log) {
+        const uint32_t* __restrict__ order, ChunkLog log, int have_start) {
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (slot >= n) return;
@@ -1686,7 +1788,7 @@ SVOX2_FWD_KERNEL void k_render_rays(
     __shared__ float log_lds[LOG ? (kBlock / kGroup) * kLogChunks * kLogWords : 1];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, STATS, false, LOG>(
-        g, o, r, rc, lane, out, STATS ? stats + 4 * ray : nullptr,
+        g, o, r, start_of(r, have_start ? rgb_out + 3 * ray : nullptr), rc, lane, out, STATS ? stats + 4 * ray : nullptr,
         colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray, &log,
         log_lds + (threadIdx.x / kGroup) * kLogChunks * kLogWords);
     if (!STATS) {
@@ -1715,7 +1817,7 @@ SVOX2_FWD_KERNEL void k_render_depth(GridView<DT> g, OptView o,
                                      const float* __restrict__ origins,
                                      const float* __restrict__ dirs,
                                      const float* __restrict__ clip, int64_t n,
-                                     float* __restrict__ depth_out) {
+                                     float* __restrict__ depth_out, int have_start) {
     const int64_t ray = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (ray >= n) return;
@@ -1724,13 +1826,14 @@ SVOX2_FWD_KERNEL void k_render_depth(GridView<DT> g, OptView o,
     Ray r;
     setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
     float depth = 0.f;
-    if (r.tmin <= r.tmax) {
-        float t = r.tmin, log_t = 0.f;
+    const float begin = have_start ? depth_out[ray] : r.tmin;
+    if (begin <= r.tmax) {
+        float t = begin, log_t = 0.f;
         bool more = true;
         int guard = 0;
         while (more && ++guard < kMaxIters) {
             Chunk c;
-            march_chunk(g, o, r, lane, t, log_t, c);
+            march_chunk(g, o, r, lane, MarchStart{t}, log_t, c);
             if (MODE == kDepthSigma) {
                 if (c.live_mask != 0) {
                     const float tj = group_bcast(c.t, __ffs(c.live_mask) - 1);
@@ -1833,7 +1936,7 @@ SVOX2_FWD_KERNEL void k_render_nvol(GridView<DT> g, OptView o, const float* __re
         int guard = 0;
         while (more && ++guard < kMaxIters) {
             Chunk c;
-            march_chunk(g, o, r, lane, t, 0.f, c);
+            march_chunk(g, o, r, lane, MarchStart{t}, 0.f, c);
             const float e = c.contrib ? __expf(-c.ws * c.sigma) : 1.f;
             int sat;
             c.weight = nvol_accumulate(lane, c.contrib, e, alpha, sat);
@@ -1887,7 +1990,7 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
         int guard = 0;
         while (more && ++guard < kMaxIters) {
             Chunk c;
-            march_chunk(g, o, r, lane, t, 0.f, c);
+            march_chunk(g, o, r, lane, MarchStart{t}, 0.f, c);
             const float e = c.contrib ? __expf(-c.ws * c.sigma) : 1.f;
             int sat;
             c.weight = nvol_accumulate(lane, c.contrib, e, alpha, sat);
@@ -1931,7 +2034,7 @@ SVOX2_BWD_KERNEL void k_render_nvol_backward(
     int guard = 0;
     while (more && ++guard < kMaxIters) {
         Chunk c;
-        march_chunk(g, o, r, lane, t, 0.f, c);
+        march_chunk(g, o, r, lane, MarchStart{t}, 0.f, c);
         const float x = __expf(-c.ws * c.sigma);
         int sat, sat2;
         c.weight = nvol_accumulate(lane, c.contrib, c.contrib ? x : 1.f, alpha, sat);
@@ -2327,7 +2430,7 @@ SVOX2_FWD_KERNEL void k_grid_weight_render(GridView<float> g, OptView o, svox2_c
 template <typename DT, int B>
 SVOX2_FWD_KERNEL void k_render_image(
         GridView<DT> g, OptView o, svox2_camera_t cam, float* __restrict__ rgb_out,
-        float* __restrict__ log_t_out) {
+        float* __restrict__ log_t_out, int have_start) {
     const int64_t ray = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     const int64_t n = static_cast<int64_t>(cam.width) * cam.height;
@@ -2341,8 +2444,9 @@ SVOX2_FWD_KERNEL void k_render_image(
     setup_ray(g, o, wo, wd, nullptr, r);
     float out[3];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
-    const float log_t = march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr,
-                                                    colour_lds + threadIdx.x / kGroup);
+    const float log_t = march_forward<DT, B, false>(
+        g, o, r, start_of(r, have_start ? rgb_out + 3 * ray : nullptr), rc, lane, out, nullptr,
+        colour_lds + threadIdx.x / kGroup);
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
     if (log_t_out != nullptr && lane == 0) log_t_out[ray] = log_t;
 }
@@ -2376,7 +2480,7 @@ SVOX2_FWD_KERNEL void k_render_tiles(const svox2_grid_t* __restrict__ grids, int
     setup_ray(g, o, wo, wd, nullptr, r);
     float out[3];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
-    march_forward<DT, B, false>(g, o, r, rc, lane, out, nullptr,
+    march_forward<DT, B, false>(g, o, r, MarchStart{r.tmin}, rc, lane, out, nullptr,
                                 colour_lds + threadIdx.x / kGroup);
     if (lane < 3) tile.rgb_out[3 * pixel + lane] = pick3(out, lane);
 }
@@ -2386,7 +2490,7 @@ SVOX2_BWD_KERNEL void k_render_backward(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
         const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n,
         const float* __restrict__ grad_out, const float* __restrict__ color_cache,
-        const uint32_t* __restrict__ order, GradOut go) {
+        const uint32_t* __restrict__ order, const float* __restrict__ begin, GradOut go) {
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (slot >= n) return;
@@ -2401,7 +2505,7 @@ SVOX2_BWD_KERNEL void k_render_backward(
     const float accum = fmaf(cc[0], gq[0], fmaf(cc[1], gq[1], cc[2] * gq[2]));
     __shared__ BwdShared sh;
     BwdRay<B> st(rc, lane, gq, accum, 0.f, &sh, go);
-    march_backward<DT, B>(g, o, r, rc, lane, st, go);
+    march_backward<DT, B>(g, o, r, rc, lane, st, go, begin != nullptr ? begin[ray] : r.tmin);
 }
 
 // One item of the replay: a ray's recorded chunks from header slot pos on, at
@@ -2531,7 +2635,7 @@ void k_render_backward_mse(
     }
     __shared__ BwdShared sh;
     BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
-    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
+    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, r.tmin, log, ray);
 }
 
 // Counting sort of the rays by descending cost in two launches: a histogram,
@@ -2838,6 +2942,38 @@ void launch_length_order(const svox2_grid_t* grid, const OptView& o, const float
     launch_cost_order(w.cost, w, n, s, 0, true);
 }
 
+// Whether a launch of n rays begins with k_march_start: it needs the cell map,
+// and samples of empty cells must not count (threshold >= 0).  Its 64 steps, one
+// read after the other, take 60 us whatever the size, which pays from about
+// 100000 rays on (65536 ordered rays: 297 us of march with or without).
+constexpr int64_t kHeadRays = 100000;
+bool march_start_pays(const svox2_grid_t* grid, const OptView& o, int64_t n) {
+    return n >= kHeadRays && grid->cell_map != nullptr && o.sigma_thresh >= 0.f;
+}
+
+// k_march_start for a ray batch (cam NULL) or an image, into out (words values
+// per ray); with an ordering workspace also the order by the remaining length.
+void launch_march_start(const svox2_grid_t* grid, const OptView& o, const svox2_camera_t* cam,
+                        const float* origins, const float* dirs, const float* clip, int64_t n,
+                        int words, float* out, const OrderWorkspace* w, hipStream_t s) {
+    const double diag = sqrt(static_cast<double>(grid->size[0]) * grid->size[0] +
+                             static_cast<double>(grid->size[1]) * grid->size[1] +
+                             static_cast<double>(grid->size[2]) * grid->size[2]);
+    const float bins = static_cast<float>((kCostBins - 2) / diag);
+    const dim3 blocks(blocks_for(n, kHeadBlock));
+    uint32_t* key = w != nullptr ? w->cost : nullptr;
+    uint32_t* clear = w != nullptr ? w->hist : nullptr;
+    if (cam != nullptr)
+        hipLaunchKernelGGL(k_march_start<true>, blocks, dim3(kHeadBlock), 0, s,
+                           make_view<float>(*grid), o, *cam, origins, dirs, clip, n, words, out,
+                           bins, key, clear);
+    else
+        hipLaunchKernelGGL(k_march_start<false>, blocks, dim3(kHeadBlock), 0, s,
+                           make_view<float>(*grid), o, svox2_camera_t{}, origins, dirs, clip, n,
+                           words, out, bins, key, clear);
+    if (w != nullptr) launch_cost_order(w->cost, *w, n, s, 0, true);
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -2932,17 +3068,20 @@ int render_rays(const svox2_grid_t* grid, const float* origins, const float* dir
     const unsigned blocks = blocks_for(n_rays * kGroup, kBlock);
     const hipStream_t s = as_stream(stream);
     OrderWorkspace w;
-    if (workspace != nullptr && n_rays >= order_min_rays()) {
-        w = order_workspace(workspace, n_rays);
+    const bool start = march_start_pays(grid, o, n_rays);
+    if (workspace != nullptr && n_rays >= order_min_rays()) w = order_workspace(workspace, n_rays);
+    if (start)
+        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, rgb_out,
+                           w.order != nullptr ? &w : nullptr, s);
+    else if (w.order != nullptr)
         launch_length_order(grid, o, origins, dirs, ray_clip, n_rays, w, s);
-    }
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
         using DT = std::remove_pointer_t<decltype(dtp)>;
         hipLaunchKernelGGL((k_render_rays<DT, B, false>), dim3(blocks), dim3(kBlock), 0, s, g, o,
                            origins, dirs, ray_clip, n_rays, rgb_out, log_transmit_out,
                            (int32_t*)nullptr, ray_cost_out, RecStream{},
-                           static_cast<const uint32_t*>(w.order), ChunkLog{});
+                           static_cast<const uint32_t*>(w.order), ChunkLog{}, start ? 1 : 0);
     });
     if (st) return st;
     if (background && (st = launch_background(grid, opt, origins, dirs, nullptr, n_rays,
@@ -2992,14 +3131,18 @@ int render_depth(const svox2_grid_t* grid, const float* origins, const float* di
     }
     const unsigned blocks = blocks_for(n_rays * kGroup, kBlock);
     const hipStream_t s = as_stream(stream);
+    const int start = march_start_pays(grid, o, n_rays) ? 1 : 0;
+    if (start)
+        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 1, depth_out,
+                           nullptr, s);
     auto launch = [&](auto g, auto dtp) {
         using DT = std::remove_pointer_t<decltype(dtp)>;
         if (mode == kDepthSigma)
             hipLaunchKernelGGL((k_render_depth<DT, kDepthSigma>), dim3(blocks), dim3(kBlock), 0,
-                               s, g, o, origins, dirs, ray_clip, n_rays, depth_out);
+                               s, g, o, origins, dirs, ray_clip, n_rays, depth_out, start);
         else
             hipLaunchKernelGGL((k_render_depth<DT, kDepthExpected>), dim3(blocks), dim3(kBlock),
-                               0, s, g, o, origins, dirs, ray_clip, n_rays, depth_out);
+                               0, s, g, o, origins, dirs, ray_clip, n_rays, depth_out, start);
     };
     if (grid->storage == SVOX2_STORAGE_BF16)
         launch(make_view<uint16_t>(*grid), (uint16_t*)nullptr);
@@ -3289,7 +3432,7 @@ extern "C" int svox2_volume_render_cuvol_stats(const svox2_grid_t* grid, const f
         hipLaunchKernelGGL((k_render_rays<DT, B, true>), dim3(blocks), dim3(kBlock), 0,
                            as_stream(stream), g, o, origins, dirs, ray_clip, n_rays,
                            (float*)nullptr, (float*)nullptr, stats_out, (uint32_t*)nullptr,
-                           RecStream{}, (const uint32_t*)nullptr, ChunkLog{});
+                           RecStream{}, (const uint32_t*)nullptr, ChunkLog{}, 0);
     });
     if (st) return st;
     return check_launch("volume_render_cuvol_stats");
@@ -3318,11 +3461,15 @@ extern "C" int svox2_volume_render_cuvol_image(const svox2_grid_t* grid,
     }
     const unsigned blocks = blocks_for(n * kGroup, kBlock);
     const svox2_camera_t c = *cam;
+    const bool start = march_start_pays(grid, o, n);
+    if (start)
+        launch_march_start(grid, o, &c, nullptr, nullptr, nullptr, n, 3, rgb_out, nullptr,
+                           as_stream(stream));
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
         using DT = std::remove_pointer_t<decltype(dtp)>;
         hipLaunchKernelGGL((k_render_image<DT, B>), dim3(blocks), dim3(kBlock), 0,
-                           as_stream(stream), g, o, c, rgb_out, log_transmit_out);
+                           as_stream(stream), g, o, c, rgb_out, log_transmit_out, start ? 1 : 0);
     });
     if (st) return st;
     if (background && (st = launch_background(grid, opt, nullptr, nullptr, &c, n,
@@ -3418,9 +3565,21 @@ extern "C" int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
         w = order_workspace(workspace, n_rays);
         launch_cost_order(ray_cost, w, n_rays, s);
     }
+    // The ordering workspace has a word per ray that an order by the caller's
+    // costs leaves free: where each ray's march begins.
+    const float* begin = nullptr;
+    if (w.order != nullptr && march_start_pays(grid, o, n_rays)) {
+        begin = reinterpret_cast<const float*>(w.cost);
+        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 1,
+                           reinterpret_cast<float*>(w.cost), nullptr, s);
+    }
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
         using DT = std::remove_pointer_t<decltype(dtp)>;
+        const bool start = background && march_start_pays(grid, o, n_rays);
+        if (start)
+            launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, bg_buf,
+                               nullptr, s);
         if (background) {
             // The reference's grid backward hands its final accum and log
             // transmittance to the background's (:1032-1064); here the grid's
@@ -3430,11 +3589,11 @@ extern "C" int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
             hipLaunchKernelGGL((k_render_rays<DT, B, false>), dim3(blocks), dim3(kBlock), 0, s,
                                g, ofg, origins, dirs, ray_clip, n_rays, bg_buf,
                                bg_buf + 3 * n_rays, (int32_t*)nullptr, (uint32_t*)nullptr,
-                               RecStream{}, (const uint32_t*)nullptr, ChunkLog{});
+                               RecStream{}, (const uint32_t*)nullptr, ChunkLog{}, start ? 1 : 0);
         }
         hipLaunchKernelGGL((k_render_backward<DT, B>), dim3(blocks), dim3(kBlock), 0, s, g, o,
                            origins, dirs, ray_clip, n_rays, grad_out, color_cache,
-                           static_cast<const uint32_t*>(w.order), go);
+                           static_cast<const uint32_t*>(w.order), begin, go);
     });
     if (st) return st;
     if (background &&
@@ -3539,7 +3698,12 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         // Large batches: the forward runs in order of segment length, then
         // the backward in order of the forward's work counts (both sorts go
         // through w.cost / w.order; the forward rewrites w.cost by ray).
-        if (w.order != nullptr) launch_length_order(grid, o, origins, dirs, ray_clip, n_rays, w, s);
+        const bool start = rs.rec == nullptr && march_start_pays(grid, o, n_rays);
+        if (start)
+            launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, rgb_out,
+                               w.order != nullptr ? &w : nullptr, s);
+        else if (w.order != nullptr)
+            launch_length_order(grid, o, origins, dirs, ray_clip, n_rays, w, s);
         const uint32_t* order = w.order;
         if (rs.rec != nullptr) {
             hipLaunchKernelGGL((k_render_rays_rec<DT, B>), dim3(blocks), dim3(kBlock), 0, s, g,
@@ -3552,11 +3716,11 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         else if (log.rec != nullptr)
             hipLaunchKernelGGL((k_render_rays<DT, B, false, true>), dim3(blocks), dim3(kBlock), 0,
                                s, g, o, origins, dirs, ray_clip, n_rays, rgb_out, lt,
-                               (int32_t*)nullptr, w.cost, rs, order, log);
+                               (int32_t*)nullptr, w.cost, rs, order, log, start ? 1 : 0);
         else
             hipLaunchKernelGGL((k_render_rays<DT, B, false>), dim3(blocks), dim3(kBlock), 0, s,
                                g, o, origins, dirs, ray_clip, n_rays, rgb_out, lt,
-                               (int32_t*)nullptr, w.cost, rs, order, log);
+                               (int32_t*)nullptr, w.cost, rs, order, log, start ? 1 : 0);
         if (background)
             bg_st = launch_background(grid, opt, origins, dirs, nullptr, n_rays, lt, rgb_out,
                                       bg_rgb, s);
