@@ -677,38 +677,34 @@ __device__ __forceinline__ uint32_t backward_cost(uint32_t work) {
     return work < static_cast<uint32_t>(kCostBins) ? work : static_cast<uint32_t>(kCostBins - 1);
 }
 
-// Run heads of a chunk: live samples whose previous live sample (in lane
-// order) is not in the same cell.  Runs are formed over the live samples
-// alone, so a chunk whose live samples are compacted into lanes 0 .. n - 1
-// (the records) has the same runs, passes and sums.
-__device__ __forceinline__ uint32_t run_heads(const Chunk& c, int lane) {
-    const uint32_t below = c.live_mask & ((1u << lane) - 1u);
-    const int prev = below ? 31 - static_cast<int>(__clz(below)) : 0;
-    const int prev_cell = __shfl(c.base, prev, kGroup);
-    return group_ballot(c.live && !(below != 0u && prev_cell == c.base));
-}
-
 // LDS of one 32-lane group for chunk_colours.
-constexpr int kColourRuns = 16;  // runs projected at a time
 struct __align__(16) ColourLds {
-    float4 at[kGroup];                 // per live sample, in order: position, weight
-    int4 links[kGroup][2];             // per run: corner links
-    float4 proj[kColourRuns][6];       // per run: 8 corners x 3 channels
-    int run[kGroup];                   // per live sample: its run
+    float4 at[kGroup];        // per live sample, in order: position, weight
+    float proj[kGroup][24];   // per run: 8 corner links, then 8 corners x 3 projections
+    int run[kGroup];          // per live sample: its run; per run, << 8: the step to it
 };
+
+// Orders this wavefront's LDS writes before its later LDS reads, and nothing else.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
 
 // Colours of a chunk's live samples.  Consecutive live samples in the same cell
 // form a run; they share the 8 corner rows, so each row is read and projected on
 // the SH basis once per run.
 // - The live samples and the runs' links go to LDS in order.
-// - lane = (run, corner), four runs per pass: the lane reads its corner's row and
-//   leaves the three projections in LDS.
+// - lane = (quarter, corner): the lane goes through its quarter of the runs, reads
+//   its corner's row and leaves the three projections in LDS.  A run's cell is
+//   mostly next to the one before it; the corners they share take the
+//   projections that are there.  The rows' bytes, 128 per corner through the
+//   CU's 64 bytes a cycle, bound this part.
 // - lane = sample: each weights its run's 8 x 3 projections trilinearly.  One
 //   pass serves up to 32 samples; with the lanes still on (run, corner), each
 //   run's samples were taken in turn and summed over the 8 corners by lane
 //   moves, about 40 instructions per sample of the longest of four runs.
-// 128x128 view of the 256^3 grid in bf16: 137 -> 94 us; 800x800 view at 512^3:
-// 1.60 -> 1.43 ms (both with the transmittance chain by lane shifts).
+// 128x128 view of the 256^3 grid in bf16: 137 -> 99 us; 800x800 view at 512^3,
+// from its first samples on: 1073 -> 1004 us for the shared corners.
 // sum receives the chunk's colour, the samples' weight * max(colour + 0.5, 0)
 // added in an order that depends on their ranks alone; with TO_LANES each live
 // lane receives its own sample's colour + 0.5 in cs.  The sums per sample are
@@ -717,59 +713,92 @@ template <typename DT, int B, bool TO_LANES>
 __device__ __forceinline__ void chunk_colours(const GridView<DT>& g, const RayCtx<B>& rc,
                                               const Chunk& c, int lane, ColourLds* sh, float* cs,
                                               float* sum) {
-    const uint32_t heads = run_heads(c, lane);
+    // Run heads: live samples whose previous live sample (in lane order) is not
+    // in the same cell.  Runs are formed over the live samples alone, so a chunk
+    // whose live samples are compacted into lanes 0 .. n - 1 (the records) has
+    // the same runs and sums.
     const uint32_t below = (1u << lane) - 1u;
-    const int rank = __popc(c.live_mask & below);
-    if (c.live) {
-        const bool head = ((heads >> lane) & 1u) != 0;
-        const int my_run = __popc(heads & below) - (head ? 0 : 1);
-        sh->at[rank] = make_float4(c.p[0], c.p[1], c.p[2], c.weight);
-        sh->run[rank] = my_run;
-        if (head) {
-            sh->links[my_run][0] = make_int4(c.lk[0], c.lk[1], c.lk[2], c.lk[3]);
-            sh->links[my_run][1] = make_int4(c.lk[4], c.lk[5], c.lk[6], c.lk[7]);
-        }
+    const uint32_t before = c.live_mask & below;
+    const int prev = before ? 31 - static_cast<int>(__clz(before)) : 0;
+    int d[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) d[a] = c.l[a] - __shfl(c.l[a], prev, kGroup);
+    const bool head = c.live && (before == 0u || (d[0] | d[1] | d[2]) != 0);
+    const uint32_t heads = group_ballot(head);
+    const int rank = __popc(before);
+    // The step to a run from the one before it: bit 6 for a neighbour cell, bits
+    // 0-2 the axes moved along, 3-5 those among them moved down.
+    int step = 0;
+    if (before != 0u && max(max(abs(d[0]), abs(d[1])), abs(d[2])) <= 1)
+        step = 64 | (d[0] != 0 ? 4 : 0) | (d[1] != 0 ? 2 : 0) | (d[2] != 0 ? 1 : 0) |
+               (d[0] < 0 ? 32 : 0) | (d[1] < 0 ? 16 : 0) | (d[2] < 0 ? 8 : 0);
+    const int my_run = __popc(heads & below) - (head ? 0 : 1);
+    if (c.live) sh->at[rank] = make_float4(c.p[0], c.p[1], c.p[2], c.weight);
+    if (c.live) sh->run[rank] = my_run;
+    wave_lds_order();
+    if (head) {
+        float* links = sh->proj[my_run];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) links[k] = __int_as_float(c.lk[k]);
+        atomicOr(&sh->run[my_run], step << 8);
     }
-    wave_lds_fence();
+    wave_lds_order();
     const int n_runs = __popc(heads);
     const bool has = lane < __popc(c.live_mask);
     const float4 q = has ? sh->at[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const int run = has ? sh->run[lane] : -1;
-    const float p[3] = {q.x, q.y, q.z};
-    float col[3] = {0.f, 0.f, 0.f};
     const int k = lane & 7;
-    for (int base = 0; base < n_runs; base += kColourRuns) {
-        const int end = min(n_runs, base + kColourRuns);
-        for (int r = base + (lane >> 3); r < end; r += 4) {
-            const int lk = reinterpret_cast<const int*>(sh->links[r])[k];
+    const int quarter = (n_runs + 3) >> 2;
+    const int first = (lane >> 3) * quarter;
+    int to = first < n_runs ? sh->run[first] >> 8 : 0;
+    int lk = first < n_runs ? __float_as_int(sh->proj[first][k]) : -1;
+    for (int i = 0; i < quarter; ++i) {
+        const int r = first + i;
+        // The next run's link and step are on their way while this one's row is
+        // read.
+        const int next = min(r + 1, n_runs - 1);
+        const int to_next = sh->run[next] >> 8;
+        const int lk_next = __float_as_int(sh->proj[next][k]);
+        wave_lds_order();  // a run's links are read before its projections take their place
+        if (r < n_runs) {
+            const int moved = to & 7, down = (to >> 3) & 7;
             float c0 = 0.f, c1 = 0.f, c2 = 0.f;
-            if (g.valid(lk)) project_row<B>(g, lk, rc.basis, c0, c1, c2);
-            float* out = reinterpret_cast<float*>(sh->proj[r - base]) + 3 * k;
+            if (i > 0 && (to & 64) && ((k ^ down) & moved) == 0) {
+                const float* from = sh->proj[r - 1] + 3 * (k ^ moved);
+                c0 = from[0];
+                c1 = from[1];
+                c2 = from[2];
+            } else if (g.valid(lk)) {
+                project_row<B>(g, lk, rc.basis, c0, c1, c2);
+            }
+            float* out = sh->proj[r] + 3 * k;
             out[0] = c0;
             out[1] = c1;
             out[2] = c2;
         }
-        wave_lds_fence();
-        if (run >= base && run < end) {
-            const float4* v4 = sh->proj[run - base];
-            float v[24];
+        wave_lds_order();
+        to = to_next;
+        lk = lk_next;
+    }
+    float col[3] = {0.f, 0.f, 0.f};
+    if (has) {
+        const float p[3] = {q.x, q.y, q.z};
+        const float4* v4 = reinterpret_cast<const float4*>(sh->proj[sh->run[lane] & 0xFF]);
+        float v[24];
 #pragma unroll
-            for (int i = 0; i < 6; ++i) {
-                const float4 x = v4[i];
-                v[4 * i] = x.x;
-                v[4 * i + 1] = x.y;
-                v[4 * i + 2] = x.z;
-                v[4 * i + 3] = x.w;
-            }
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                float t[8];
-#pragma unroll
-                for (int kk = 0; kk < 8; ++kk) t[kk] = v[3 * kk + a] * corner_weight(kk, p);
-                col[a] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
-            }
+        for (int i = 0; i < 6; ++i) {
+            const float4 x = v4[i];
+            v[4 * i] = x.x;
+            v[4 * i + 1] = x.y;
+            v[4 * i + 2] = x.z;
+            v[4 * i + 3] = x.w;
         }
-        wave_lds_fence();  // the next runs' projections, or the caller, take the space
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            float t[8];
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) t[kk] = v[3 * kk + a] * corner_weight(kk, p);
+            col[a] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        }
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -777,6 +806,7 @@ __device__ __forceinline__ void chunk_colours(const GridView<DT>& g, const RayCt
         sum[a] = group_lane(group_scan(has ? q.w * fmaxf(shown, 0.f) : 0.f), 31);
         if (TO_LANES) cs[a] = __shfl(shown, c.live ? rank : 0, kGroup);
     }
+    wave_lds_fence();  // the caller may take the space
 }
 
 // Chunk log of the fused call: the forward writes the placement of each of a
@@ -792,6 +822,21 @@ struct ChunkLog {
 };
 constexpr int kLogChunks = 16;
 constexpr int kLogWords = 36;
+constexpr int kLogStage = 4;  // chunks staged in LDS
+static_assert(kLogChunks % kLogStage == 0, "the stage is written out when full");
+
+// Writes the staged chunks first .. first + count - 1 of a ray's log out.
+__device__ __forceinline__ void write_log(const ChunkLog& log, const float* stage, int64_t ray,
+                                          int first, int count, int lane) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int i = 0; i < count; ++i) {
+        const float* src = stage + i * kLogWords;
+        float* dst = log.rec + (ray * kLogChunks + first + i) * kLogWords;
+        dst[lane] = src[lane];
+        if (lane < 2) dst[32 + lane] = src[32 + lane];
+    }
+}
 
 // Record stream of the fused call: the forward appends, per ray, a header and
 // one 96-byte record per contributing sample of each chunk; the backward
@@ -907,10 +952,11 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                 march_chunk(g, o, r, lane, at, log_t, c);
                 const int n_live = __popc(c.live_mask);
                 if (LOG && n_chunks < static_cast<uint32_t>(kLogChunks)) {
-                    // Staged in LDS and written out when the ray ends: global
-                    // stores here would hold up the next chunk's loads (a load's
-                    // wait also waits for every earlier store).
-                    float* rec = log_lds + n_chunks * kLogWords;
+                    // Staged in LDS and written out a few chunks at a time: a
+                    // global store holds up the next chunk's loads (a load's
+                    // wait also waits for every earlier store), and LDS for all
+                    // 16 chunks leaves room for 13 wavefronts per CU of 20.
+                    float* rec = log_lds + n_chunks % kLogStage * kLogWords;
                     rec[lane] = c.t;
                     if (lane == 0) {
                         rec[32] = __int_as_float(c.n_place);
@@ -918,6 +964,9 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                     }
                     log_more = c.more;
                     log_next_t = c.next_t;
+                    if (n_chunks % kLogStage == kLogStage - 1)
+                        write_log(*log, log_lds, ray, static_cast<int>(n_chunks) + 1 - kLogStage,
+                                  kLogStage, lane);
                 }
                 ++n_chunks;
                 if (RECORD && n_live > 0) {
@@ -1065,13 +1114,8 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
     }
     if (LOG) {
         const int n_logged = static_cast<int>(min(n_chunks, static_cast<uint32_t>(kLogChunks)));
-        wave_lds_fence();
-        for (int ci = 0; ci < n_logged; ++ci) {
-            const float* src = log_lds + ci * kLogWords;
-            float* dst = log->rec + (ray * kLogChunks + ci) * kLogWords;
-            dst[lane] = src[lane];
-            if (lane < 2) dst[32 + lane] = src[32 + lane];
-        }
+        const int staged = n_logged % kLogStage;
+        write_log(*log, log_lds, ray, n_logged - staged, staged, lane);
         if (lane == 0)
             log->head[ray] = make_int4(n_logged, log_more ? 1 : 0, __float_as_int(log_next_t), 0);
     }
@@ -1649,7 +1693,9 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
             c.p[0] = a.x;
             c.p[1] = a.y;
             c.p[2] = a.z;
-            c.base = __float_as_int(a.w);
+            c.l[0] = __float_as_int(b.x);
+            c.l[1] = __float_as_int(b.y);
+            c.l[2] = __float_as_int(b.z);
             c.weight = b.w;
             c.lk[0] = __float_as_int(c2.x);
             c.lk[1] = __float_as_int(c2.y);
@@ -1661,7 +1707,7 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
             c.lk[7] = __float_as_int(d.w);
         } else {
             c.p[0] = c.p[1] = c.p[2] = 0.f;
-            c.base = -1;
+            c.l[0] = c.l[1] = c.l[2] = 0;
             c.weight = 0.f;
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk) c.lk[kk] = -1;
@@ -1785,12 +1831,12 @@ SVOX2_FWD_KERNEL void k_render_rays(
     float out[3];
     uint32_t cost = 0;
     // LDS staging of this group's chunk log (used when LOG).
-    __shared__ float log_lds[LOG ? (kBlock / kGroup) * kLogChunks * kLogWords : 1];
+    __shared__ float log_lds[LOG ? (kBlock / kGroup) * kLogStage * kLogWords : 1];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, STATS, false, LOG>(
         g, o, r, start_of(r, have_start ? rgb_out + 3 * ray : nullptr), rc, lane, out, STATS ? stats + 4 * ray : nullptr,
         colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray, &log,
-        log_lds + (threadIdx.x / kGroup) * kLogChunks * kLogWords);
+        log_lds + (threadIdx.x / kGroup) * kLogStage * kLogWords);
     if (!STATS) {
         if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
         if (log_t_out != nullptr && lane == 0) log_t_out[ray] = log_t;
