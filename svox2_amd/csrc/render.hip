@@ -1452,10 +1452,10 @@ __device__ __forceinline__ void scatter_chunk(const GridView<DT>& g, const GradO
 template <typename DT, int B, bool PREFETCH = true>
 __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptView& o,
                                                const Ray& r, const RayCtx<B>& rc, int lane,
-                                               BwdRay<B>& st, const GradOut& go, float begin,
+                                               BwdRay<B>& st, const GradOut& go,
                                                ChunkLog log_v = ChunkLog{},
                                                int64_t ray = 0) {
-    if (!(begin <= r.tmax)) return;
+    if (r.tmin > r.tmax) return;
     // Chunks the forward logged are evaluated from their placement.
     int n_logged = 0;
     bool log_more = false;
@@ -1484,7 +1484,7 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
         int nl[3];
         load_corner_links(g, lane, sample_cell(g, r, nt, np, nl), nmask, nlk);
     }
-    float t = begin;
+    float t = r.tmin;
     float log_t = 0.f;
     int guard = 0;
     bool more = true;
@@ -1748,8 +1748,8 @@ constexpr int kHeadLanes = 4;
 template <bool IMAGE>
 __global__ __launch_bounds__(kHeadBlock) void k_march_start(
         GridView<float> g, OptView o, svox2_camera_t cam, const float* __restrict__ origins,
-        const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n, int words,
-        float* __restrict__ out, float bins_per_voxel, uint32_t* __restrict__ key,
+        const float* __restrict__ dirs, int64_t n, int words, float* __restrict__ out,
+        float bins_per_voxel, uint32_t* __restrict__ key,
         uint32_t* __restrict__ clear) {
     if (key != nullptr && blockIdx.x == 0)  // both histograms of the ordering workspace
         for (int b = threadIdx.x; b < 2 * kCostBins; b += kHeadBlock) clear[b] = 0u;
@@ -1766,7 +1766,7 @@ __global__ __launch_bounds__(kHeadBlock) void k_march_start(
         }
     }
     Ray r;
-    setup_ray(g, o, wo, wd, clip ? clip + 2 * i : nullptr, r);
+    setup_ray(g, o, wo, wd, nullptr, r);
     MarchStart at{r.tmin};
     // The wavefront walks on while enough of its lanes do, kHeadSteps at most;
     // the rest is left to the march, which may begin anywhere on the walk (a ray
@@ -2536,7 +2536,7 @@ SVOX2_BWD_KERNEL void k_render_backward(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
         const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n,
         const float* __restrict__ grad_out, const float* __restrict__ color_cache,
-        const uint32_t* __restrict__ order, const float* __restrict__ begin, GradOut go) {
+        const uint32_t* __restrict__ order, GradOut go) {
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (slot >= n) return;
@@ -2551,7 +2551,7 @@ SVOX2_BWD_KERNEL void k_render_backward(
     const float accum = fmaf(cc[0], gq[0], fmaf(cc[1], gq[1], cc[2] * gq[2]));
     __shared__ BwdShared sh;
     BwdRay<B> st(rc, lane, gq, accum, 0.f, &sh, go);
-    march_backward<DT, B>(g, o, r, rc, lane, st, go, begin != nullptr ? begin[ray] : r.tmin);
+    march_backward<DT, B>(g, o, r, rc, lane, st, go);
 }
 
 // One item of the replay: a ray's recorded chunks from header slot pos on, at
@@ -2681,7 +2681,7 @@ void k_render_backward_mse(
     }
     __shared__ BwdShared sh;
     BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
-    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, r.tmin, log, ray);
+    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
 }
 
 // Counting sort of the rays by descending cost in two launches: a histogram,
@@ -2991,17 +2991,18 @@ void launch_length_order(const svox2_grid_t* grid, const OptView& o, const float
 // Whether a launch of n rays begins with k_march_start: it needs the cell map,
 // and samples of empty cells must not count (threshold >= 0).  Its 64 steps, one
 // read after the other, take 60 us whatever the size, which pays from about
-// 100000 rays on (65536 ordered rays: 297 us of march with or without).
+// 100000 rays on (65536 ordered rays: 297 us of march with or without).  Clipped
+// rays are left out: they are shorter, and 262144 of them lost 20 us by it.
 constexpr int64_t kHeadRays = 100000;
-bool march_start_pays(const svox2_grid_t* grid, const OptView& o, int64_t n) {
-    return n >= kHeadRays && grid->cell_map != nullptr && o.sigma_thresh >= 0.f;
+bool march_start_pays(const svox2_grid_t* grid, const OptView& o, int64_t n, const float* clip) {
+    return n >= kHeadRays && clip == nullptr && grid->cell_map != nullptr && o.sigma_thresh >= 0.f;
 }
 
 // k_march_start for a ray batch (cam NULL) or an image, into out (words values
 // per ray); with an ordering workspace also the order by the remaining length.
 void launch_march_start(const svox2_grid_t* grid, const OptView& o, const svox2_camera_t* cam,
-                        const float* origins, const float* dirs, const float* clip, int64_t n,
-                        int words, float* out, const OrderWorkspace* w, hipStream_t s) {
+                        const float* origins, const float* dirs, int64_t n, int words,
+                        float* out, const OrderWorkspace* w, hipStream_t s) {
     const double diag = sqrt(static_cast<double>(grid->size[0]) * grid->size[0] +
                              static_cast<double>(grid->size[1]) * grid->size[1] +
                              static_cast<double>(grid->size[2]) * grid->size[2]);
@@ -3011,12 +3012,12 @@ void launch_march_start(const svox2_grid_t* grid, const OptView& o, const svox2_
     uint32_t* clear = w != nullptr ? w->hist : nullptr;
     if (cam != nullptr)
         hipLaunchKernelGGL(k_march_start<true>, blocks, dim3(kHeadBlock), 0, s,
-                           make_view<float>(*grid), o, *cam, origins, dirs, clip, n, words, out,
+                           make_view<float>(*grid), o, *cam, origins, dirs, n, words, out,
                            bins, key, clear);
     else
         hipLaunchKernelGGL(k_march_start<false>, blocks, dim3(kHeadBlock), 0, s,
-                           make_view<float>(*grid), o, svox2_camera_t{}, origins, dirs, clip, n,
-                           words, out, bins, key, clear);
+                           make_view<float>(*grid), o, svox2_camera_t{}, origins, dirs, n, words, out,
+                           bins, key, clear);
     if (w != nullptr) launch_cost_order(w->cost, *w, n, s, 0, true);
 }
 
@@ -3114,10 +3115,10 @@ int render_rays(const svox2_grid_t* grid, const float* origins, const float* dir
     const unsigned blocks = blocks_for(n_rays * kGroup, kBlock);
     const hipStream_t s = as_stream(stream);
     OrderWorkspace w;
-    const bool start = march_start_pays(grid, o, n_rays);
+    const bool start = march_start_pays(grid, o, n_rays, ray_clip);
     if (workspace != nullptr && n_rays >= order_min_rays()) w = order_workspace(workspace, n_rays);
     if (start)
-        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, rgb_out,
+        launch_march_start(grid, o, nullptr, origins, dirs, n_rays, 3, rgb_out,
                            w.order != nullptr ? &w : nullptr, s);
     else if (w.order != nullptr)
         launch_length_order(grid, o, origins, dirs, ray_clip, n_rays, w, s);
@@ -3177,9 +3178,9 @@ int render_depth(const svox2_grid_t* grid, const float* origins, const float* di
     }
     const unsigned blocks = blocks_for(n_rays * kGroup, kBlock);
     const hipStream_t s = as_stream(stream);
-    const int start = march_start_pays(grid, o, n_rays) ? 1 : 0;
+    const int start = march_start_pays(grid, o, n_rays, ray_clip) ? 1 : 0;
     if (start)
-        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 1, depth_out,
+        launch_march_start(grid, o, nullptr, origins, dirs, n_rays, 1, depth_out,
                            nullptr, s);
     auto launch = [&](auto g, auto dtp) {
         using DT = std::remove_pointer_t<decltype(dtp)>;
@@ -3507,9 +3508,9 @@ extern "C" int svox2_volume_render_cuvol_image(const svox2_grid_t* grid,
     }
     const unsigned blocks = blocks_for(n * kGroup, kBlock);
     const svox2_camera_t c = *cam;
-    const bool start = march_start_pays(grid, o, n);
+    const bool start = march_start_pays(grid, o, n, nullptr);
     if (start)
-        launch_march_start(grid, o, &c, nullptr, nullptr, nullptr, n, 3, rgb_out, nullptr,
+        launch_march_start(grid, o, &c, nullptr, nullptr, n, 3, rgb_out, nullptr,
                            as_stream(stream));
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
@@ -3611,20 +3612,12 @@ extern "C" int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
         w = order_workspace(workspace, n_rays);
         launch_cost_order(ray_cost, w, n_rays, s);
     }
-    // The ordering workspace has a word per ray that an order by the caller's
-    // costs leaves free: where each ray's march begins.
-    const float* begin = nullptr;
-    if (w.order != nullptr && march_start_pays(grid, o, n_rays)) {
-        begin = reinterpret_cast<const float*>(w.cost);
-        launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 1,
-                           reinterpret_cast<float*>(w.cost), nullptr, s);
-    }
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
         constexpr int B = decltype(b)::value;
         using DT = std::remove_pointer_t<decltype(dtp)>;
-        const bool start = background && march_start_pays(grid, o, n_rays);
+        const bool start = background && march_start_pays(grid, o, n_rays, ray_clip);
         if (start)
-            launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, bg_buf,
+            launch_march_start(grid, o, nullptr, origins, dirs, n_rays, 3, bg_buf,
                                nullptr, s);
         if (background) {
             // The reference's grid backward hands its final accum and log
@@ -3639,7 +3632,7 @@ extern "C" int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
         }
         hipLaunchKernelGGL((k_render_backward<DT, B>), dim3(blocks), dim3(kBlock), 0, s, g, o,
                            origins, dirs, ray_clip, n_rays, grad_out, color_cache,
-                           static_cast<const uint32_t*>(w.order), begin, go);
+                           static_cast<const uint32_t*>(w.order), go);
     });
     if (st) return st;
     if (background &&
@@ -3744,9 +3737,9 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         // Large batches: the forward runs in order of segment length, then
         // the backward in order of the forward's work counts (both sorts go
         // through w.cost / w.order; the forward rewrites w.cost by ray).
-        const bool start = rs.rec == nullptr && march_start_pays(grid, o, n_rays);
+        const bool start = rs.rec == nullptr && march_start_pays(grid, o, n_rays, ray_clip);
         if (start)
-            launch_march_start(grid, o, nullptr, origins, dirs, ray_clip, n_rays, 3, rgb_out,
+            launch_march_start(grid, o, nullptr, origins, dirs, n_rays, 3, rgb_out,
                                w.order != nullptr ? &w : nullptr, s);
         else if (w.order != nullptr)
             launch_length_order(grid, o, origins, dirs, ray_clip, n_rays, w, s);
