@@ -669,8 +669,7 @@ __device__ __forceinline__ void project_row(const GridView<uint16_t>& g, int lk,
 // (no half-wave idles behind a long ray) and the longest rays no longer finish
 // last on an otherwise idle device.  Smaller batches run in one round, where
 // pairing the longest rays in the same waves only slows them, and keep the
-// input order.  When the backward replays recorded samples instead, its
-// work is per record and per recorded chunk, and that count is the key.
+// input order.
 constexpr int kCostBins = 1024;
 
 __device__ __forceinline__ uint32_t backward_cost(uint32_t work) {
@@ -847,32 +846,24 @@ __device__ __forceinline__ void write_log(const ChunkLog& log, const float* stag
 // state[r] = 1 when the ray's stream is complete, 2 when the overflow region
 // ran out (the backward then re-marches the ray).
 //
-// Long rays are replayed in segments: a ray with at least kRecSplitMin
-// recorded chunks lists its segments m >= 1 in seg_list (one reservation per
-// ray, seg_cap entries in all) and sets split; seg[r * (kRecSegs - 1) + m -
-// 1] holds the header slot of its recorded chunk m * kRecSegChunks (-1 past
-// its end), where segment m's backward starts.
+// The recorded chunks of all rays are listed in clist; the backward replays each
+// by itself.
 struct RecStream {
     float4* __restrict__ rec;
     int32_t* __restrict__ state;
     // Counters, one per partition of rays (ray % parts), so that no single
     // address takes every ray's atomic: [p] overflow slots taken of opart,
-    // [kRecParts + p] segment list entries of spart, [2 kRecParts + p] chunk
-    // list entries of cpart; partition p owns every parts-th overflow block and
-    // the p-th slice of each list.
+    // [kRecParts + p] chunk list entries of cpart; partition p owns every
+    // parts-th overflow block and the p-th slice of the list.
     uint32_t* __restrict__ next_block;
     int parts;
-    int64_t opart, spart, cpart;
-    int32_t* __restrict__ seg;
-    int32_t* __restrict__ split;        // per ray: 1 if its segments are listed, else -1
-    int2* __restrict__ seg_list;        // (ray, segment m >= 1), or (-1, -1)
-    int64_t seg_cap;
+    int64_t opart, cpart;
     int64_t fixed;                      // slots per ray in the fixed region
     int64_t overflow_base;              // first overflow slot
     int64_t overflow_slots;             // slots in the overflow region
-    // Deferred colours: the recorded chunks of rays whose colours are formed
-    // by k_rec_colours.
-    int2* __restrict__ clist;           // (ray, header slot), or (-1, -1)
+    // The recorded chunks, whose colours k_rec_colours forms.
+    uint2* __restrict__ clist;          // (ray | number in its ray << kRayBits, header slot),
+                                        // or slot kNoSlot
     float4* __restrict__ chunk_rgb;     // per entry: the chunk's colour
     float4* __restrict__ ray_info;      // per ray: (first entry, entries, background term)
     int64_t clist_cap;
@@ -880,10 +871,9 @@ struct RecStream {
 constexpr int kRecBlock = 64;  // >= 32 records + header + the end/jump header
 constexpr int kRecParts = 64;  // counter partitions at most
 constexpr int kDeferChunks = 64;  // recorded chunks a ray can list for deferred colours
-constexpr int64_t kDeferCap = 8;  // chunk list entries per ray of the batch
-constexpr int kRecSegChunks = 1;  // recorded chunks per replay segment
-constexpr int kRecSegs = 24;      // segments of a split ray (the last runs to its end)
-constexpr int kRecSplitMin = 2 * kRecSegChunks;  // recorded chunks that make a ray split
+constexpr int64_t kDeferCap = 9;  // chunk list entries per ray of the batch
+constexpr int kRayBits = 26;  // rays of a recorded batch; kDeferChunks numbers fit above them
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 
 // A chunk of n records occupies slots slot .. slot + n (the header, then n
 // records), stored field-major after the header's slot: field j (0..5) of
@@ -932,7 +922,6 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
     float total[3] = {0.f, 0.f, 0.f};  // colour composited so far
     uint32_t n_iter = 0, n_eval = 0, n_hit = 0;
     uint32_t n_chunks = 0;
-    uint32_t n_live_all = 0, n_live_chunks = 0;  // replay work (recording only)
     Fnv fnv;
     float log_t = 0.f;
     bool defer = DEFER;
@@ -940,7 +929,7 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
         if (DEFER && attempt == 1) {  // the deferred march did not fit
             defer = false;
             total[0] = total[1] = total[2] = 0.f;
-            n_chunks = n_live_all = n_live_chunks = 0;
+            n_chunks = 0;
         }
         log_t = 0.f;
         if (start.t <= r.tmax) {
@@ -969,16 +958,7 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                                   kLogStage, lane);
                 }
                 ++n_chunks;
-                if (RECORD && n_live > 0) {
-                    n_live_all += n_live;
-                    ++n_live_chunks;
-                }
                 if (n_live > 0) {
-                    // Recorded chunk k = n_rec_chunks opens replay segment
-                    // k / kRecSegChunks when k is a multiple of kRecSegChunks.
-                    const bool seg_start = RECORD && rec_ok && n_rec_chunks > 0 &&
-                                           n_rec_chunks % kRecSegChunks == 0 &&
-                                           n_rec_chunks / kRecSegChunks < kRecSegs;
                     float cs[3] = {0.f, 0.f, 0.f};
                     if (!defer) {
                         float sum[3];
@@ -1010,9 +990,6 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                         if (DEFER && defer && n_rec_chunks >= kDeferChunks) rec_ok = false;
                         if (rec_ok) {
                             const int k = n_rec_chunks++;
-                            if (seg_start && lane == 0)  // a replay segment may start here
-                                rs->seg[ray * (kRecSegs - 1) + k / kRecSegChunks - 1] =
-                                    static_cast<int32_t>(cur);
                             if (DEFER && defer && lane == 0) slot_lds[k] = static_cast<int32_t>(cur);
                             if (lane == 0) put_header(rs->rec, cur, n_live, 0);
                             if (c.live) {
@@ -1055,7 +1032,7 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
             const int part = static_cast<int>(ray % rs->parts);
             int local = 0;
             if (lane == 0)
-                local = static_cast<int>(atomicAdd(rs->next_block + 2 * kRecParts + part,
+                local = static_cast<int>(atomicAdd(rs->next_block + kRecParts + part,
                                                    static_cast<uint32_t>(n_rec_chunks)));
             local = __shfl(local, 0, kGroup);
             const bool fits = static_cast<int64_t>(local) + n_rec_chunks <= rs->cpart;
@@ -1064,7 +1041,8 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
             for (int k = lane; k < n_rec_chunks; k += kGroup) {
                 if (static_cast<int64_t>(local) + k < rs->cpart)
                     rs->clist[static_cast<int64_t>(first) + k] =
-                        fits ? make_int2(static_cast<int>(ray), slot_lds[k]) : make_int2(-1, -1);
+                        make_uint2(static_cast<uint32_t>(ray) | (static_cast<uint32_t>(k) << kRayBits),
+                                   fits ? static_cast<uint32_t>(slot_lds[k]) : kNoSlot);
             }
             if (!fits) {
                 rec_ok = false;
@@ -1081,36 +1059,12 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
     const float tb = __expf(log_t) * o.bg;
 #pragma unroll
     for (int a = 0; a < 3; ++a) out[a] = total[a] + tb;
-    // A replayed backward works per record and per recorded chunk, a
-    // re-marching one per chunk.
-    if (cost != nullptr)
-        *cost = backward_cost(RECORD ? n_live_all + 4u * n_live_chunks : n_chunks);
+    if (cost != nullptr) *cost = backward_cost(n_chunks);
     if (RECORD) {
-        // A long ray lists its segments m >= 1 for the replay (one reservation).
-        int n_seg = 1;
-        if (rec_ok && n_rec_chunks >= kRecSplitMin)
-            n_seg = min((n_rec_chunks + kRecSegChunks - 1) / kRecSegChunks, kRecSegs);
-        const int part = static_cast<int>(ray % rs->parts);
-        int local = 0;
-        if (lane == 0 && n_seg > 1)
-            local = static_cast<int>(atomicAdd(rs->next_block + kRecParts + part,
-                                               static_cast<uint32_t>(n_seg - 1)));
-        local = __shfl(local, 0, kGroup);
-        const bool listed = n_seg > 1 && static_cast<int64_t>(local) + n_seg - 1 <= rs->spart;
-        for (int m = 1 + lane; m < n_seg; m += kGroup) {
-            const int64_t l = static_cast<int64_t>(local) + m - 1;
-            if (l < rs->spart)
-                rs->seg_list[part * rs->spart + l] =
-                    listed ? make_int2(static_cast<int>(ray), m) : make_int2(-1, -1);
-        }
         if (lane == 0) {
             if (rec_ok) put_header(rs->rec, cur, -1, 0);
             rs->state[ray] = rec_ok ? 1 : 2;
-            rs->split[ray] = listed ? 1 : -1;
         }
-        const int m_end = 1 + lane;  // segments the ray does not have
-        if (m_end < kRecSegs && (!rec_ok || m_end * kRecSegChunks >= n_rec_chunks))
-            rs->seg[ray * (kRecSegs - 1) + m_end - 1] = -1;
     }
     if (LOG) {
         const int n_logged = static_cast<int>(min(n_chunks, static_cast<uint32_t>(kLogChunks)));
@@ -1539,49 +1493,37 @@ __device__ __forceinline__ void march_backward(const GridView<DT>& g, const OptV
     st.sc.flush_all(g, go, lane);
 }
 
-// Backward of one ray from its record stream (the fused call's forward wrote
-// every contributing sample with its colour and transmittance): no link,
-// density or SH reads, only the records and the gradient scatter.  Starts at
-// the header slot pos and replays at most max_chunks recorded chunks.
+// Backward of one recorded chunk (its header at slot pos): no link, density or
+// SH reads, only the records and the gradient scatter.  Nothing is read after
+// the scatter: a load's wait also waits for every atomic before it.
 template <typename DT, int B>
-__device__ __forceinline__ void replay_backward(const GridView<DT>& g, const RecStream& rs,
-                                                int64_t pos, int max_chunks, int lane,
-                                                BwdRay<B>& st, const GradOut& go) {
-    int chunks = 0;
-    for (int guard = 0; guard < kMaxIters; ++guard) {
-        const float4 h = rs.rec[6 * pos];
-        const int n = __float_as_int(h.x);
-        if (n < 0) break;
-        if (n == 0) {
-            pos = __float_as_int(h.y);
-            continue;
-        }
-        if (chunks++ == max_chunks) break;  // the next segment's first chunk
-        const bool live = lane < n;
-        float p[3] = {0.f, 0.f, 0.f}, cs[3] = {0.f, 0.f, 0.f};
-        int l[3] = {0, 0, 0}, lk[8];
-        float weight = 0.f, lt_after = 0.f, ws = 0.f, sigma = 0.f;
-        if (live) {
-            const float4* q = rec_field0(rs.rec, pos) + lane;
-            const float4 a = q[0], b = q[n], c2 = q[2 * n], d = q[3 * n], e = q[4 * n], f = q[5 * n];
-            p[0] = a.x; p[1] = a.y; p[2] = a.z;
-            l[0] = __float_as_int(b.x); l[1] = __float_as_int(b.y); l[2] = __float_as_int(b.z);
-            weight = b.w;
-            lk[0] = __float_as_int(c2.x); lk[1] = __float_as_int(c2.y);
-            lk[2] = __float_as_int(c2.z); lk[3] = __float_as_int(c2.w);
-            lk[4] = __float_as_int(d.x); lk[5] = __float_as_int(d.y);
-            lk[6] = __float_as_int(d.z); lk[7] = __float_as_int(d.w);
-            cs[0] = e.x; cs[1] = e.y; cs[2] = e.z; lt_after = e.w;
-            ws = f.x; sigma = f.y;
-        } else {
+__device__ __forceinline__ void replay_chunk(const GridView<DT>& g, const RecStream& rs,
+                                             int64_t pos, int lane, BwdRay<B>& st,
+                                             const GradOut& go) {
+    const int n = __float_as_int(rs.rec[6 * pos].x);
+    const bool live = lane < n;
+    float p[3] = {0.f, 0.f, 0.f}, cs[3] = {0.f, 0.f, 0.f};
+    int l[3] = {0, 0, 0}, lk[8];
+    float weight = 0.f, lt_after = 0.f, ws = 0.f, sigma = 0.f;
+    if (live) {
+        const float4* q = rec_field0(rs.rec, pos) + lane;
+        const float4 a = q[0], b = q[n], c2 = q[2 * n], d = q[3 * n], e = q[4 * n], f = q[5 * n];
+        p[0] = a.x; p[1] = a.y; p[2] = a.z;
+        l[0] = __float_as_int(b.x); l[1] = __float_as_int(b.y); l[2] = __float_as_int(b.z);
+        weight = b.w;
+        lk[0] = __float_as_int(c2.x); lk[1] = __float_as_int(c2.y);
+        lk[2] = __float_as_int(c2.z); lk[3] = __float_as_int(c2.w);
+        lk[4] = __float_as_int(d.x); lk[5] = __float_as_int(d.y);
+        lk[6] = __float_as_int(d.z); lk[7] = __float_as_int(d.w);
+        cs[0] = e.x; cs[1] = e.y; cs[2] = e.z; lt_after = e.w;
+        ws = f.x; sigma = f.y;
+    } else {
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) lk[kk] = -1;
-        }
-        const uint32_t live_mask = n >= 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
-        scatter_chunk<DT, B>(g, go, st, lane, live, live_mask, p, l, lk, cs, weight, lt_after,
-                             ws, sigma);
-        pos += n + 1;
+        for (int kk = 0; kk < 8; ++kk) lk[kk] = -1;
     }
+    const uint32_t live_mask = n >= 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
+    scatter_chunk<DT, B>(g, go, st, lane, live, live_mask, p, l, lk, cs, weight, lt_after, ws,
+                         sigma);
     st.sc.flush_all(g, go, lane);
 }
 
@@ -1634,8 +1576,8 @@ template <typename DT, int B>
 SVOX2_REC_KERNEL void k_render_rays_rec(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
         const float* __restrict__ dirs, const float* __restrict__ clip, int64_t n,
-        float* __restrict__ rgb_out, float* __restrict__ log_t_out,
-        uint32_t* __restrict__ cost_out, RecStream rs, const uint32_t* __restrict__ order) {
+        float* __restrict__ rgb_out, float* __restrict__ log_t_out, RecStream rs,
+        const uint32_t* __restrict__ order) {
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (slot >= n) return;
@@ -1646,17 +1588,15 @@ SVOX2_REC_KERNEL void k_render_rays_rec(
     Ray r;
     setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
     float out[3];
-    uint32_t cost = 0;
     // LDS staging of this group's recorded chunk header slots.
     __shared__ int32_t slot_lds[(kBlock / kGroup) * kDeferChunks];
     __shared__ ColourLds colour_lds[kBlock / kGroup];
     const float log_t = march_forward<DT, B, false, true, false, true>(
-        g, o, r, MarchStart{r.tmin}, rc, lane, out, nullptr, colour_lds + threadIdx.x / kGroup, cost_out != nullptr ? &cost : nullptr, &rs, ray,
+        g, o, r, MarchStart{r.tmin}, rc, lane, out, nullptr, colour_lds + threadIdx.x / kGroup, nullptr, &rs, ray,
         nullptr, nullptr, slot_lds + (threadIdx.x / kGroup) * kDeferChunks);
     // A ray whose chunks were listed gets its colour from k_rec_colours.
     if (lane < 3) rgb_out[3 * ray + lane] = pick3(out, lane);
     if (log_t_out != nullptr && lane == 0) log_t_out[ray] = log_t;
-    if (cost_out != nullptr && lane == 0) cost_out[ray] = cost;
 }
 
 // Colours of the chunks the recording forward listed, one group per chunk
@@ -1677,12 +1617,12 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
     const int64_t per_part = static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) / rs.parts;
     const int64_t part = gid % rs.parts;
     if (gid >= per_part * rs.parts) return;
-    const int64_t entries = min(static_cast<int64_t>(rs.next_block[2 * kRecParts + part]), rs.cpart);
+    const int64_t entries = min(static_cast<int64_t>(rs.next_block[kRecParts + part]), rs.cpart);
     for (int64_t l = gid / rs.parts; l < entries; l += per_part) {
         const int64_t j = part * rs.cpart + l;
-        const int2 e = rs.clist[j];
-        if (e.x < 0) continue;  // entries of a ray whose list did not fit
-        const int64_t ray = e.x, slot = e.y;
+        const uint2 e = rs.clist[j];
+        if (e.y == kNoSlot) continue;  // entries of a ray whose list did not fit
+        const int64_t ray = e.x & ((1u << kRayBits) - 1u), slot = e.y;
         const int n = __float_as_int(rs.rec[6 * slot].x);
         Chunk c;
         c.live = lane < n;
@@ -2554,19 +2494,17 @@ SVOX2_BWD_KERNEL void k_render_backward(
     march_backward<DT, B>(g, o, r, rc, lane, st, go);
 }
 
-// One item of the replay: a ray's recorded chunks from header slot pos on, at
-// most max_chunks of them.  seg_chunk: recorded chunks before them (segments
-// m >= 1 of a split ray), or -1 from the ray's start; that item writes the
-// ray's colour.
+// One item of the replay: a ray's recorded chunk number `chunk`, its header at
+// slot pos.  Chunk 0's item writes the ray's colour.
 template <typename DT, int B>
 __device__ __forceinline__ void replay_item(
         const GridView<DT>& g, const float* dirs, const float* rgb_gt, float* rgb_out,
         const float* log_t_fwd, float beta_per_ray, float sparsity, float norm,
-        const GradOut& go, const RecStream& rs, int lane, int64_t ray, int64_t pos,
-        int max_chunks, int seg_chunk, BwdShared* sh) {
+        const GradOut& go, const RecStream& rs, int lane, int64_t ray, int64_t pos, int chunk,
+        BwdShared* sh) {
     const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
     const RayCtx<B> rc(wd);
-    // The ray's colour, and the colour composited before the segment.
+    // The ray's colour, and the colour composited before the chunk.
     const float4 info = rs.ray_info[ray];
     const int first = __float_as_int(info.x), cnt = __float_as_int(info.y);
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -2574,7 +2512,7 @@ __device__ __forceinline__ void replay_item(
     const float4 v1 = lane + kGroup < cnt ? rs.chunk_rgb[first + kGroup + lane] : zero4;
     float c3[3] = {0.f, 0.f, 0.f}, before[3] = {0.f, 0.f, 0.f};
     for (int k = 0; k < cnt; ++k) {
-        if (k == seg_chunk) {
+        if (k == chunk) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) before[c] = c3[c];
         }
@@ -2589,60 +2527,51 @@ __device__ __forceinline__ void replay_item(
         c3[c] += info.z;
         gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
     }
-    if (seg_chunk < 0 && lane < 3) rgb_out[3 * ray + lane] = pick3(c3, lane);
+    if (chunk == 0 && lane < 3) rgb_out[3 * ray + lane] = pick3(c3, lane);
     float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
     if (beta_per_ray > 0.f) {
         const float tin = __expf(log_t_fwd[ray]);
         accum += beta_per_ray * (1.f - tin / (1.f - tin + 1e-3f));
     }
-    if (seg_chunk >= 0)  // accum after the samples before the segment
+    if (chunk > 0)  // accum after the samples before the chunk
         accum -= fmaf(before[0], gq[0], fmaf(before[1], gq[1], before[2] * gq[2]));
     BwdRay<B> st(rc, lane, gq, accum, sparsity, sh, go);
-    replay_backward<DT, B>(g, rs, pos, max_chunks, lane, st, go);
+    replay_chunk<DT, B>(g, rs, pos, lane, st, go);
 }
 
 // Backward of the fused MSE step for the rays whose samples the forward
 // recorded (state 1): the same gradient as k_render_backward_mse, from the
 // records, in a kernel without the march code (fewer registers, more waves).
 // The ray's colour is the sum of its chunk colours (k_rec_colours) in march
-// order plus the background term, as the forward forms it; the group of item
-// < n writes it to rgb_out.  A segment m >= 1 of a split ray starts from the
-// colour composited before its first chunk.
+// order plus the background term, as the forward forms it; rays without a
+// recorded chunk have theirs from the forward.  A segment starts from the colour
+// composited before its first chunk.
+//
+// The gradient atomics bound it: the card takes 19.9 G atomic requests a second,
+// whatever their scope, locality or width up to 64 bytes, so a row is two, and
+// 65536 rays at 512^3 visit 2.9M rows (1.4 visits a row): 291 us of the kernel's
+// 330 us; 4096 rays of a dense 64^3 grid 1.7M, 170 of 172 us.  Longer segments
+// would save the 8 rows a chunk ends with, but a group is then held by its own
+// atomics: 2 chunks each 335 us, 4 361 us, 8 388 us.
 template <typename DT, int B>
 SVOX2_REPLAY_KERNEL void k_render_backward_replay(
-        GridView<DT> g, const float* __restrict__ dirs, int64_t n,
-        const float* __restrict__ rgb_gt, float* __restrict__ rgb_out,
-        const float* __restrict__ log_t_fwd, float beta_per_ray, float sparsity, float norm,
-        const uint32_t* __restrict__ order, GradOut go, RecStream rs) {
-    const int64_t item = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
+        GridView<DT> g, const float* __restrict__ dirs, const float* __restrict__ rgb_gt,
+        float* __restrict__ rgb_out, const float* __restrict__ log_t_fwd, float beta_per_ray,
+        float sparsity, float norm, GradOut go, RecStream rs) {
+    const int64_t gid = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     __shared__ BwdShared sh;
-    if (item < n) {  // a ray from its start; a split ray's first segment only
-        const int64_t ray = order != nullptr ? static_cast<int64_t>(order[item]) : item;
-        if (rs.state[ray] != 1) return;  // re-marched by k_render_backward_mse
+    // Each partition's entries go round its share of the groups.
+    const int64_t per_part = static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) / rs.parts;
+    const int64_t part = gid % rs.parts;
+    if (gid >= per_part * rs.parts) return;
+    const int64_t entries = min(static_cast<int64_t>(rs.next_block[kRecParts + part]), rs.cpart);
+    for (int64_t l = gid / rs.parts; l < entries; l += per_part) {
+        const uint2 e = rs.clist[part * rs.cpart + l];
+        const int chunk = static_cast<int>(e.x >> kRayBits);
+        if (e.y == kNoSlot) continue;
         replay_item<DT, B>(g, dirs, rgb_gt, rgb_out, log_t_fwd, beta_per_ray, sparsity, norm, go,
-                           rs, lane, ray, ray * rs.fixed,
-                           rs.split[ray] >= 0 ? kRecSegChunks : kMaxIters, -1, &sh);
-        return;
-    }
-    // Listed segments m >= 1 of split rays: each partition's entries go round
-    // its share of the remaining groups.
-    const int64_t sg = item - n;
-    const int64_t per_part =
-        (static_cast<int64_t>(gridDim.x) * (kBlock / kGroup) - n) / rs.parts;
-    const int64_t part = sg % rs.parts;
-    if (sg >= per_part * rs.parts) return;
-    const int64_t entries = min(static_cast<int64_t>(rs.next_block[kRecParts + part]), rs.spart);
-    for (int64_t l = sg / rs.parts; l < entries; l += per_part) {
-        const int2 sm = rs.seg_list[part * rs.spart + l];
-        if (sm.x < 0) continue;  // entries of a ray whose segments did not fit
-        const int64_t ray = sm.x;
-        const int m = sm.y;
-        const int64_t pos = rs.seg[ray * (kRecSegs - 1) + m - 1];
-        if (pos < 0) continue;  // the ray ends before this segment
-        replay_item<DT, B>(g, dirs, rgb_gt, rgb_out, log_t_fwd, beta_per_ray, sparsity, norm, go,
-                           rs, lane, ray, pos, m < kRecSegs - 1 ? kRecSegChunks : kMaxIters,
-                           m * kRecSegChunks, &sh);
+                           rs, lane, e.x & ((1u << kRayBits) - 1u), e.y, chunk, &sh);
     }
 }
 
@@ -2650,7 +2579,9 @@ SVOX2_REPLAY_KERNEL void k_render_backward_replay(
 // forward colours (render_ray_backward_kernel with grad_out_is_rgb,
 // render_lerp_kernel_cuvol.cu:735-741), plus the beta term from the forward's
 // final log transmittance (:257-262) and the Cauchy sparsity term (:345-348).
-template <typename DT, int B, int WAVES>
+// SCAN (record path): the rays are those whose records did not fit (state 2),
+// which each group looks for among 32 rays at a time.
+template <typename DT, int B, int WAVES, bool SCAN>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES)))
 void k_render_backward_mse(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
@@ -2660,28 +2591,43 @@ void k_render_backward_mse(
         const uint32_t* __restrict__ order, GradOut go, RecStream rs, ChunkLog log) {
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
-    if (slot >= n) return;
-    const int64_t ray = order != nullptr ? static_cast<int64_t>(order[slot]) : slot;
-    if (rs.rec != nullptr && rs.state[ray] == 1) return;  // replayed by k_render_backward_replay
-    const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
-    const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
-    const RayCtx<B> rc(wd);
-    Ray r;
-    setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
-    float c3[3], gq[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        c3[c] = rgb[3 * ray + c];
-        gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
-    }
-    float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
-    if (beta_per_ray > 0.f) {
-        const float tin = __expf(log_t_fwd[ray]);
-        accum += beta_per_ray * (1.f - tin / (1.f - tin + 1e-3f));
-    }
     __shared__ BwdShared sh;
-    BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
-    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
+    int64_t base = SCAN ? slot * kGroup : slot, ray = 0;
+    uint32_t todo = 0u;
+    for (;;) {
+        if (SCAN) {
+            const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+            while (todo == 0u) {  // the next 32 rays
+                if (base >= n) return;
+                todo = group_ballot(base + lane < n && rs.state[min(base + lane, n - 1)] == 2);
+                base += stride;
+            }
+            ray = base - stride + __ffs(todo) - 1;
+            todo &= todo - 1u;
+        } else {
+            if (slot >= n) return;
+            ray = order != nullptr ? static_cast<int64_t>(order[slot]) : slot;
+        }
+        const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
+        const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
+        const RayCtx<B> rc(wd);
+        Ray r;
+        setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
+        float c3[3], gq[3];
+    #pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            c3[c] = rgb[3 * ray + c];
+            gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
+        }
+        float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
+        if (beta_per_ray > 0.f) {
+            const float tin = __expf(log_t_fwd[ray]);
+            accum += beta_per_ray * (1.f - tin / (1.f - tin + 1e-3f));
+        }
+        BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
+        march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
+        if (!SCAN) return;
+    }
 }
 
 // Counting sort of the rays by descending cost in two launches: a histogram,
@@ -2820,30 +2766,22 @@ OrderWorkspace order_workspace(void* ws, int64_t n) {
 // per-ray state (n words), the overflow counter, and the record slots (n *
 // (kRecFixed + kRecOverflow) slots of 96 bytes).
 constexpr int64_t kRecFixed = 8;      // slots per ray in the fixed region
-constexpr int64_t kRecOverflow = 40;  // overflow slots per ray
+constexpr int64_t kRecOverflow = 41;  // overflow slots per ray
 constexpr int64_t kRecSlotBytes = 96;
 
 inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 
-// Segment list entries: three extra segments per ray of the batch (rays
-// whose segments do not fit are replayed whole).
-int64_t seg_cap_of(int64_t n) { return 3 * n; }
-
-// [order | state (n) | seg (n (kRecSegs - 1)) | split (n) | seg_list | counters |
+// [order | state (n) | counters |
 //  ray_info (n) | clist (kDeferCap n) | chunk_rgb (kDeferCap n) | records]
 size_t fused_workspace_bytes(int64_t n) {
     const int64_t order = static_cast<int64_t>(order_workspace_bytes(n));
     const int64_t state = align256(4 * n);
-    const int64_t seg = align256(4 * n * (kRecSegs - 1));
-    const int64_t split = align256(4 * n);
-    const int64_t list = align256(8 * seg_cap_of(n));
-    const int64_t counter = align256(4 * 3 * kRecParts);
+    const int64_t counter = align256(4 * 4 * kRecParts);
     const int64_t info = align256(16 * n);
     const int64_t clist = align256(8 * kDeferCap * n);
     const int64_t crgb = align256(16 * kDeferCap * n);
     const int64_t recs = n * (kRecFixed + kRecOverflow) * kRecSlotBytes;
-    return static_cast<size_t>(order + state + seg + split + list + counter + info + clist +
-                               crgb + recs);
+    return static_cast<size_t>(order + state + counter + info + clist + crgb + recs);
 }
 
 // Fused-call workspace with the chunk log (batches that re-march): the
@@ -2857,13 +2795,13 @@ size_t logged_workspace_bytes(int64_t n) {
 }
 
 // Record capacity beyond the least (4096 rays of a dense 64^3 grid hold about
-// 130 contributing samples each: with the least 48 slots a ray most were marched
+// 130 contributing samples each: with the least 49 slots a ray most were marched
 // twice and re-marched by the backward, 0.43 ms a step; with room for all of
 // them 0.30 ms): a workspace of more bytes scales the
 // overflow slots and the two lists by the same factor (in 1/64).
 int64_t record_scale(size_t bytes, int64_t n) {
     const int64_t least = static_cast<int64_t>(fused_workspace_bytes(n));
-    const int64_t per_ray = 8 * 3 + 24 * kDeferCap + kRecOverflow * kRecSlotBytes;
+    const int64_t per_ray = 24 * kDeferCap + kRecOverflow * kRecSlotBytes;
     const int64_t extra = static_cast<int64_t>(bytes) - least - 4 * 256;  // alignment
     // Header slots are int32: at most 2^31 - 1 slots.
     const int64_t most = 64 * (INT32_MAX - n * kRecFixed) / (n * kRecOverflow);
@@ -2884,18 +2822,11 @@ RecStream record_stream(void* ws, size_t bytes, int64_t n) {
     RecStream rs{};
     rs.state = reinterpret_cast<int32_t*>(p);
     p += align256(4 * n);
-    rs.seg = reinterpret_cast<int32_t*>(p);
-    p += align256(4 * n * (kRecSegs - 1));
-    rs.split = reinterpret_cast<int32_t*>(p);
-    p += align256(4 * n);
-    rs.seg_list = reinterpret_cast<int2*>(p);
-    rs.seg_cap = seg_cap_of(n) * scale / 64;
-    p += align256(8 * rs.seg_cap);
     rs.next_block = reinterpret_cast<uint32_t*>(p);
-    p += align256(4 * 3 * kRecParts);
+    p += align256(4 * 4 * kRecParts);
     rs.ray_info = reinterpret_cast<float4*>(p);
     p += align256(16 * n);
-    rs.clist = reinterpret_cast<int2*>(p);
+    rs.clist = reinterpret_cast<uint2*>(p);
     rs.clist_cap = kDeferCap * n * scale / 64;
     p += align256(8 * rs.clist_cap);
     rs.chunk_rgb = reinterpret_cast<float4*>(p);
@@ -2914,7 +2845,6 @@ RecStream record_stream(void* ws, size_t bytes, int64_t n) {
     const int64_t per_part = scale >= 4 * 64 ? 64 : (n < 16384 ? n : 1024);
     rs.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n / per_part, kRecParts)));
     rs.opart = rs.overflow_slots / kRecBlock / rs.parts * kRecBlock;
-    rs.spart = rs.seg_cap / rs.parts;
     rs.cpart = rs.clist_cap / rs.parts;
     return rs;
 }
@@ -3728,7 +3658,7 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         workspace_bytes >= fused_workspace_bytes(n_rays)) {
         rs = record_stream(workspace, workspace_bytes, n_rays);
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kSortBlock), 0, s,
-                           reinterpret_cast<uint32_t*>(rs.next_block), 3 * kRecParts);
+                           reinterpret_cast<uint32_t*>(rs.next_block), 2 * kRecParts);
     }
     int bg_st = 0;
     st = dispatch(grid, [&](auto g, auto b, auto dtp) {
@@ -3746,8 +3676,7 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         const uint32_t* order = w.order;
         if (rs.rec != nullptr) {
             hipLaunchKernelGGL((k_render_rays_rec<DT, B>), dim3(blocks), dim3(kBlock), 0, s, g,
-                               o, origins, dirs, ray_clip, n_rays, rgb_out, lt, w.cost, rs,
-                               order);
+                               o, origins, dirs, ray_clip, n_rays, rgb_out, lt, rs, order);
             hipLaunchKernelGGL((k_rec_colours<DT, B>),
                                dim3(blocks_for(std::min(rs.clist_cap, 2 * n_rays) * kGroup, kBlock)),
                                dim3(kBlock), 0, s, g, dirs, rs);
@@ -3763,24 +3692,30 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
         if (background)
             bg_st = launch_background(grid, opt, origins, dirs, nullptr, n_rays, lt, rgb_out,
                                       bg_rgb, s);
+        if (rs.rec != nullptr) {
+            // The chunks are alike, and only the device knows how many there are.
+            hipLaunchKernelGGL((k_render_backward_replay<DT, B>),
+                               dim3(blocks_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s, g,
+                               dirs, rgb_gt, rgb_out, lt, beta, sparsity_loss, norm, go, rs);
+            hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES_FEW, true>),
+                               dim3(blocks_for(n_rays, kBlock)), dim3(kBlock), 0, s, g, o,
+                               origins, dirs, ray_clip, n_rays, rgb_gt, rgb_out, lt, beta,
+                               sparsity_loss, norm, static_cast<const uint32_t*>(nullptr), go,
+                               rs, log);
+            return;
+        }
         // The key kernel cleared both histograms; this sort uses the second.
         if (w.order != nullptr) launch_cost_order(w.cost, w, n_rays, s, 1, true);
-        if (rs.rec != nullptr)
-            hipLaunchKernelGGL((k_render_backward_replay<DT, B>),
-                               dim3(blocks_for((n_rays + seg_cap_of(n_rays)) * kGroup,
-                                               kBlock)),
-                               dim3(kBlock), 0, s, g, dirs, n_rays, rgb_gt, rgb_out, lt, beta,
-                               sparsity_loss, norm, static_cast<const uint32_t*>(w.order), go, rs);
         // Batches of up to 4 device fills use the 3-wave build.
         if (n_rays <= 4 * order_min_rays())
-            hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES_FEW>), dim3(blocks),
-                               dim3(kBlock), 0, s, g, o, origins, dirs, ray_clip, n_rays, rgb_gt,
-                               rgb_out, lt, beta, sparsity_loss, norm,
+            hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES_FEW, false>),
+                               dim3(blocks), dim3(kBlock), 0, s, g, o, origins, dirs, ray_clip,
+                               n_rays, rgb_gt, rgb_out, lt, beta, sparsity_loss, norm,
                                static_cast<const uint32_t*>(w.order), go, rs, log);
         else
-            hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES>), dim3(blocks),
-                               dim3(kBlock), 0, s, g, o, origins, dirs, ray_clip, n_rays, rgb_gt,
-                               rgb_out, lt, beta, sparsity_loss, norm,
+            hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES, false>),
+                               dim3(blocks), dim3(kBlock), 0, s, g, o, origins, dirs, ray_clip,
+                               n_rays, rgb_gt, rgb_out, lt, beta, sparsity_loss, norm,
                                static_cast<const uint32_t*>(w.order), go, rs, log);
     });
     if (st) return st;
