@@ -1752,6 +1752,13 @@ __device__ __forceinline__ MarchStart start_of(const Ray& r, const float* found)
     return MarchStart{found[0], place & 0xFF, place >> 8};
 }
 
+// Whether k_march_start saw the whole ray and found no sample with rows: the
+// kernel then writes that ray's result at once.  Set up (its direction's
+// reciprocals are rounded from doubles) and taken into the march, such rays were
+// 77 us of the 1030 us of an 800x800 image at 512^3, 13 us of 519 of its depth
+// and 12 us of 425 of 200003 rays in bf16.
+__device__ __forceinline__ bool nothing_met(const float* found) { return found[0] == INFINITY; }
+
 template <typename DT, int B, bool STATS, bool LOG = false>
 SVOX2_FWD_KERNEL void k_render_rays(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
@@ -1763,6 +1770,15 @@ SVOX2_FWD_KERNEL void k_render_rays(
     const int lane = threadIdx.x % kGroup;
     if (slot >= n) return;
     const int64_t ray = order != nullptr ? static_cast<int64_t>(order[slot]) : slot;
+    if (!STATS && have_start && nothing_met(rgb_out + 3 * ray)) {
+        if (lane < 3) rgb_out[3 * ray + lane] = 0.f + o.bg;
+        if (lane == 0) {
+            if (log_t_out != nullptr) log_t_out[ray] = 0.f;
+            if (cost_out != nullptr) cost_out[ray] = backward_cost(0);
+            if (LOG) log.head[ray] = make_int4(0, 0, 0, 0);
+        }
+        return;
+    }
     const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
     const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
     const RayCtx<B> rc(wd);
@@ -1807,6 +1823,10 @@ SVOX2_FWD_KERNEL void k_render_depth(GridView<DT> g, OptView o,
     const int64_t ray = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     if (ray >= n) return;
+    if (have_start && nothing_met(depth_out + ray)) {
+        if (lane == 0) depth_out[ray] = 0.f;
+        return;
+    }
     const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
     const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
     Ray r;
@@ -2421,6 +2441,11 @@ SVOX2_FWD_KERNEL void k_render_image(
     const int lane = threadIdx.x % kGroup;
     const int64_t n = static_cast<int64_t>(cam.width) * cam.height;
     if (ray >= n) return;
+    if (have_start && nothing_met(rgb_out + 3 * ray)) {
+        if (lane < 3) rgb_out[3 * ray + lane] = 0.f + o.bg;
+        if (log_t_out != nullptr && lane == 0) log_t_out[ray] = 0.f;
+        return;
+    }
     const int ix = static_cast<int>(ray % cam.width);
     const int iy = static_cast<int>(ray / cam.width);
     float wd[3], wo[3];

@@ -1,7 +1,8 @@
 """Kernel variants at the sizes where their tiling can go wrong: point sets
 around the sampler's 16 points per wavefront and its cell-map thresholds, MSI
 backgrounds whose layers and columns do not fill the scatter's 8-layer window or
-wrap onto slots of the same parity."""
+wrap onto slots of the same parity, launches on both sides of the ray count
+from which a march's start is searched by a lane per ray."""
 import numpy as np
 import pytest
 import torch
@@ -146,3 +147,49 @@ def test_fused_record_capacity(gpu, dense64, n, factor):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
     for x, y in zip(a[2:], b[2:]):
         assert (x - y).abs().max() <= 1e-5 * x.abs().max()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [100000, 100033])
+def test_march_start(gpu, dtype, n):
+    """The start searched for, and rays that it finds nothing on written without
+    a march: colours have the same bits as in calls of fewer rays, which march
+    from the grid's edge.  Depths sum the same terms in chunks that begin
+    elsewhere: two float32 sums, each a tree of 5 levels and at most 20 chunks
+    (96^3: under 640 samples), differ by at most 2 * 25 * 2^-24 of the depth."""
+    gen = torch.Generator().manual_seed(n)
+    spec = scenes.BlobSpec(3, (0.1, 0.15), (20.0, 20.0))
+    grid = _grid(scenes.make_blob_grid(96, spec, gen), gpu, dtype)
+    origins = torch.randn(n, 3, generator=gen)
+    origins = origins / origins.norm(dim=1, keepdim=True) * 2.5
+    dirs = torch.rand(n, 3, generator=gen) * 1.6 - 0.8 - origins
+    dirs = dirs / dirs.norm(dim=1, keepdim=True)
+    origins, dirs = origins.to(gpu), dirs.to(gpu)
+    with torch.no_grad():
+        rays = svox2_amd.Rays(origins, dirs)
+        rgb, depth = grid.volume_render(rays), grid.volume_render_depth(rays)
+        parts = [svox2_amd.Rays(origins[i:i + 30000].contiguous(), dirs[i:i + 30000].contiguous())
+                 for i in range(0, n, 30000)]
+        assert torch.equal(rgb, torch.cat([grid.volume_render(p) for p in parts]))
+        want = torch.cat([grid.volume_render_depth(p) for p in parts])
+        assert ((depth - want).abs() <= 50 * 2.0 ** -24 * want).all()
+    assert 0.2 < (depth == 0).float().mean() < 0.98
+
+
+def test_march_start_image(gpu):
+    """An image of 317 x 331 pixels against its rays in smaller calls."""
+    gen = torch.Generator().manual_seed(1)
+    spec = scenes.BlobSpec(3, (0.1, 0.15), (20.0, 20.0))
+    grid = _grid(scenes.make_blob_grid(96, spec, gen), gpu)
+    c2w = torch.eye(4)
+    c2w[2, 3] = -2.5
+    cam = svox2_amd.Camera(c2w.to(gpu), 400.0, 400.0, width=317, height=331)
+    with torch.no_grad():
+        img = grid.volume_render_image(cam).view(-1, 3)
+        rays = cam.gen_rays()
+        want = torch.cat([grid.volume_render(svox2_amd.Rays(rays.origins[i:i + 30000],
+                                                            rays.dirs[i:i + 30000]))
+                          for i in range(0, img.size(0), 30000)])
+    # The camera's rays are formed in the kernel: float32 rounding apart.
+    assert (img - want).abs().max() <= 2e-4
+    assert (img == grid.opt.background_brightness).all(1).float().mean() > 0.2
