@@ -20,6 +20,7 @@ from collections import OrderedDict
 from typing import Optional, Tuple
 
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 __all__ = [
     "SparseGridSpec", "RaysSpec", "CameraSpec", "RenderOptions", "GridOutputGrads",
@@ -452,9 +453,10 @@ def _grid_struct(g: SparseGridSpec, need_sh: bool = True, need_map: bool = True,
 
 
 # Cell maps by links tensor: (device, address, shape, version, rows, accel
-# epoch) -> (map, stream it was built on, event after the build).  The accel
-# epoch counts in-place accel_dist_prop calls, which write through a raw pointer
-# and so do not bump the tensor version.
+# epoch) -> (map, stream it was built on, event after the build, weak reference
+# to the links' storage: once that is gone, another tensor may have the address).
+# The accel epoch counts in-place accel_dist_prop calls, which write through a raw
+# pointer and so do not bump the tensor version.
 _CELL_MAPS: "OrderedDict[tuple, tuple]" = OrderedDict()
 _CELL_MAP_CACHE = 4
 _ACCEL_EPOCH: dict = {}
@@ -466,9 +468,9 @@ def _cached_cell_map(links: torch.Tensor, rows: int, build: bool = True
            _ACCEL_EPOCH.get((links.device.index, links.data_ptr()), 0))
     stream = torch.cuda.current_stream(links.device)
     found = _CELL_MAPS.get(key)
-    if found is not None:
+    if found is not None and not found[3].expired():
         _CELL_MAPS.move_to_end(key)
-        cmap, built_on, built = found
+        cmap, built_on, built, _ = found
         if stream != built_on and not torch.cuda.is_current_stream_capturing():
             # Another stream's map: wait for its build, and keep its memory
             # until this stream's work is done.
@@ -484,7 +486,7 @@ def _cached_cell_map(links: torch.Tensor, rows: int, build: bool = True
     # Drop stale maps of the same links tensor, then the oldest ones.
     for k in [k for k in _CELL_MAPS if k[:3] == key[:3]]:
         del _CELL_MAPS[k]
-    _CELL_MAPS[key] = (cmap, stream, built)
+    _CELL_MAPS[key] = (cmap, stream, built, StorageWeakRef(links.untyped_storage()))
     while len(_CELL_MAPS) > _CELL_MAP_CACHE:
         _CELL_MAPS.popitem(last=False)
     return cmap

@@ -10,7 +10,7 @@ import torch
 import oracle.oracle as O
 import svox2_amd
 from svox2_amd import _C, scenes
-from tests.conftest import host_grid
+from tests.conftest import assert_grad_close, host_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -193,3 +193,70 @@ def test_march_start_image(gpu):
     # The camera's rays are formed in the kernel: float32 rounding apart.
     assert (img - want).abs().max() <= 2e-4
     assert (img == grid.opt.background_brightness).all(1).float().mean() > 0.2
+
+
+@pytest.mark.parametrize("width,height,batch", [(8, 4, 0), (8, 4, -1), (0, 4, 5), (8, 4, 2.5)])
+def test_depth_image_refuses(gpu, dense64, width, height, batch):
+    """Batches that hold no ray stay refused, though the image is one launch."""
+    grid = _grid(dense64[4], gpu)
+    cam = svox2_amd.Camera(torch.eye(4, device=gpu), 10.0, 10.0, width=width, height=height)
+    with pytest.raises((ValueError, RuntimeError, TypeError)):
+        grid.volume_render_depth_image(cam, batch_size=batch)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 33, 65])
+def test_nvol_ray_counts(gpu, n):
+    """Few and odd rays through both forms of the nvol backward: the fused colours
+    are the forward's bits, the gradients the oracle's to the shared tolerances."""
+    gen = torch.Generator().manual_seed(n)
+    sc = scenes.make_blob_grid(24, scenes.BlobSpec(4, (0.2, 0.2), (20.0, 20.0)), gen)
+    grid = _grid(sc, gpu)
+    grid.opt.backend = "nvol"
+    hg = host_grid(sc, links=grid.links.cpu().numpy())
+    o, d = scenes.sphere_rays(n, gen, radius=1.8, target=0.4)
+    rays = svox2_amd.Rays(o.to(gpu), d.to(gpu))
+    gt = torch.rand(n, 3, generator=gen)
+    spec, opt = grid._to_cpp(), grid.opt._to_cpp()
+    rgb_f = _C.volume_render_nvol(spec, rays._to_cpp(), opt)
+    gout = ((rgb_f.cpu().double() - gt.double()) * (2.0 / (3 * n))).numpy()
+    op = grid.opt
+    opts = O.Opts(op.background_brightness, op.step_size, op.sigma_thresh, op.stop_thresh,
+                  op.near_clip, op.use_spheric_clip, op.last_sample_opaque)
+    rgd, rgs, rmask = O.nvol_grads_fp64(hg, o.numpy(), d.numpy(), opts, gout)
+    for fused in (False, True):
+        gd, gs, _, _ = grid._get_data_grads()
+        gd.zero_()
+        gs.zero_()
+        mask = torch.zeros(gd.size(0), dtype=torch.bool, device=gpu)
+        holder = _C.GridOutputGrads()
+        holder.grad_density_out, holder.grad_sh_out, holder.mask_out = gd, gs, mask
+        if fused:
+            rgb = torch.empty(n, 3, device=gpu)
+            _C.volume_render_nvol_fused(spec, rays._to_cpp(), opt, gt.to(gpu), 0.0, 0.0, rgb,
+                                        holder)
+            assert torch.equal(rgb, rgb_f)
+        else:
+            _C.volume_render_nvol_backward(spec, rays._to_cpp(), opt,
+                                           torch.from_numpy(gout).float().to(gpu), rgb_f, holder)
+        assert_grad_close(gd.cpu().numpy().reshape(-1), rgd, "grad density")
+        assert_grad_close(gs.cpu().numpy(), rgs, "grad sh")
+        assert np.array_equal(mask.cpu().numpy(), rmask)
+
+
+def test_cell_map_follows_its_links(gpu):
+    """Links allocated where others were freed get a cell map of their own."""
+    gen = torch.Generator().manual_seed(5)
+    sc = scenes.make_blob_grid(64, scenes.BlobSpec(4, (0.1, 0.1), (20.0, 20.0)), gen)
+    grid = _grid(sc, gpu)
+    pts = (torch.rand(1 << 19, 3, generator=gen) * 2 - 1).to(gpu)
+    spec = grid._to_cpp()
+    for links in (grid.links.clone(), grid.links.flip(0).clone()):
+        spec.links = torch.empty_like(links)
+        at = spec.links.data_ptr()
+        spec.links.copy_(links)
+        del links
+        spec.cell_map = None
+        got = _C.sample_grid(spec, pts, True)
+        spec.cell_map = False
+        assert all(torch.equal(a, b) for a, b in zip(got, _C.sample_grid(spec, pts, True))), at
+        spec.links = None
