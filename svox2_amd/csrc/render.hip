@@ -6,23 +6,24 @@
 // 32 consecutive samples on the 32 lanes, so the corner links and densities of
 // all of them are fetched by two waves of independent loads instead of one
 // dependent round trip per sample, and the transmittance chain is replayed in
-// registers.  Colours of the live samples are then gathered four samples at a
-// time with lane = (sample, corner): each lane reads one contiguous SH row and
-// projects it on the SH basis; the 8 corners are summed with lane shuffles.
+// registers.  The live samples' colours follow cell by cell: lane = (cell,
+// corner) reads one contiguous SH row and projects it on the SH basis, then
+// lane = sample weights its cell's projections.
 //
-// The backward pass rematerialises the same chunks, forms every live sample's
-// gradient scalars sample-parallel (the reference's running `accum` becomes a
-// prefix sum over the chunk), and adds them in sample order into registers
-// with lane = (corner, R/G/B/density): a ray that stays in a cell, or moves to
-// a neighbour (the shared corners are kept, a lane permutation), accumulates
-// without memory traffic; a corner it leaves is flushed with one no-return
-// atomic instruction covering the corner's 27 SH channels and its density
-// (one 128-byte row in the interleaved layout).
+// The backward pass takes each chunk's live samples from the forward's records,
+// places them from its log or marches again, forms their gradient scalars
+// sample-parallel (the reference's running `accum` becomes a prefix sum over
+// the chunk), and adds them in sample order into registers with lane = gradient
+// column: a ray that stays in a cell, or moves to a neighbour (the grid points
+// the two share keep their registers), accumulates without memory traffic; a
+// grid point it leaves is flushed with one no-return atomic instruction covering
+// its 27 SH channels and its density (one 128-byte row in the interleaved
+// layout, two atomic requests; the card takes about 20 G of them a second).
 //
 // Launches use 64-thread workgroups (one wavefront), so the hardware refills a
-// CU as soon as any wavefront's two rays end.  The fused call records each
-// ray's chunk count in the forward and, for large batches, runs the backward
-// over the rays in descending order of it.
+// CU as soon as any wavefront's two rays end.  Large batches run in descending
+// order of the rays' lengths (forward) and chunk counts (backward), and very
+// large ones begin with a lane-per-ray search for each march's first sample.
 //
 // Semantics follow the reference kernels: trace_ray_cuvol
 // (svox2/csrc/render_lerp_kernel_cuvol.cu:30-120), trace_ray_cuvol_backward
@@ -1679,7 +1680,7 @@ __global__ __launch_bounds__(kBlock) void k_rec_colours(GridView<DT> g,
 // key (may be NULL): the ray's order key, its length from there on.
 //
 // 800x800 view at 512^3: the march 1434 -> 1090 us, this kernel 90 us; 200003
-// rays in bf16: 675 -> 440 and 70 us.  Walked to the end, grazing rays hold it
+// rays in bf16: 675 -> 440 and 70 us (each march before its later changes).  Walked to the end, grazing rays hold it
 // for 616 us; at most 48, 64 and 128 steps give 1205, 1179 and 1203 us in all.
 constexpr int kHeadBlock = 256;
 constexpr int kHeadSteps = 64;
@@ -1972,7 +1973,7 @@ SVOX2_FWD_KERNEL void k_render_nvol(GridView<DT> g, OptView o, const float* __re
 // backward's register scatter.  Two marches with 8 density atomics per sample
 // and pass and 27 per sample and corner for the colours, sample by sample, after
 // a forward of its own, took 590 + 136 us for 30000 rays at 256^3; this kernel
-// 370 us.
+// 370 us, 312 us since the march and the colours are cheaper.
 template <typename DT, int B, bool FUSED>
 SVOX2_BWD_KERNEL void k_render_nvol_backward(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
@@ -2569,8 +2570,8 @@ __device__ __forceinline__ void replay_item(
 // records, in a kernel without the march code (fewer registers, more waves).
 // The ray's colour is the sum of its chunk colours (k_rec_colours) in march
 // order plus the background term, as the forward forms it; rays without a
-// recorded chunk have theirs from the forward.  A segment starts from the colour
-// composited before its first chunk.
+// recorded chunk have theirs from the forward.  A chunk starts from the colour
+// composited before it.
 //
 // The gradient atomics bound it: the card takes 19.9 G atomic requests a second,
 // whatever their scope, locality or width up to 64 bytes, so a row is two, and
@@ -2946,7 +2947,8 @@ void launch_length_order(const svox2_grid_t* grid, const OptView& o, const float
 // Whether a launch of n rays begins with k_march_start: it needs the cell map,
 // and samples of empty cells must not count (threshold >= 0).  Its 64 steps, one
 // read after the other, take 60 us whatever the size, which pays from about
-// 100000 rays on (65536 ordered rays: 297 us of march with or without).  Clipped
+// 100000 rays on (65536 ordered rays: 297 us of march with or without; a call for
+// a 256x256 image at 512^3 269 us without, 306 with).  Clipped
 // rays are left out: they are shorter, and 262144 of them lost 20 us by it.
 constexpr int64_t kHeadRays = 100000;
 bool march_start_pays(const svox2_grid_t* grid, const OptView& o, int64_t n, const float* clip) {
