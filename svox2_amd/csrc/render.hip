@@ -2605,9 +2605,11 @@ SVOX2_REPLAY_KERNEL void k_render_backward_replay(
 // forward colours (render_ray_backward_kernel with grad_out_is_rgb,
 // render_lerp_kernel_cuvol.cu:735-741), plus the beta term from the forward's
 // final log transmittance (:257-262) and the Cauchy sparsity term (:345-348).
-// SCAN (record path): the rays are those whose records did not fit (state 2),
-// which each group looks for among 32 rays at a time.
-template <typename DT, int B, int WAVES, bool SCAN>
+// REST (record path): only the rays whose records did not fit (state 2).  A group
+// per ray, though there are mostly none (11 us of 670 for 65536 rays): where many
+// do not fit, a group that looks for them among 32 rays marches them one by one
+// (65536 rays through the middle of a 256^3 grid: 3.6 ms a step against 2.1).
+template <typename DT, int B, int WAVES, bool REST>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(WAVES)))
 void k_render_backward_mse(
         GridView<DT> g, OptView o, const float* __restrict__ origins,
@@ -2618,42 +2620,27 @@ void k_render_backward_mse(
     const int64_t slot = (static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x) / kGroup;
     const int lane = threadIdx.x % kGroup;
     __shared__ BwdShared sh;
-    int64_t base = SCAN ? slot * kGroup : slot, ray = 0;
-    uint32_t todo = 0u;
-    for (;;) {
-        if (SCAN) {
-            const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
-            while (todo == 0u) {  // the next 32 rays
-                if (base >= n) return;
-                todo = group_ballot(base + lane < n && rs.state[min(base + lane, n - 1)] == 2);
-                base += stride;
-            }
-            ray = base - stride + __ffs(todo) - 1;
-            todo &= todo - 1u;
-        } else {
-            if (slot >= n) return;
-            ray = order != nullptr ? static_cast<int64_t>(order[slot]) : slot;
-        }
-        const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
-        const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
-        const RayCtx<B> rc(wd);
-        Ray r;
-        setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
-        float c3[3], gq[3];
-    #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            c3[c] = rgb[3 * ray + c];
-            gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
-        }
-        float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
-        if (beta_per_ray > 0.f) {
-            const float tin = __expf(log_t_fwd[ray]);
-            accum += beta_per_ray * (1.f - tin / (1.f - tin + 1e-3f));
-        }
-        BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
-        march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
-        if (!SCAN) return;
+    if (slot >= n) return;
+    const int64_t ray = order != nullptr ? static_cast<int64_t>(order[slot]) : slot;
+    if (REST && rs.state[ray] != 2) return;
+    const float wo[3] = {origins[3 * ray], origins[3 * ray + 1], origins[3 * ray + 2]};
+    const float wd[3] = {dirs[3 * ray], dirs[3 * ray + 1], dirs[3 * ray + 2]};
+    const RayCtx<B> rc(wd);
+    Ray r;
+    setup_ray(g, o, wo, wd, clip ? clip + 2 * ray : nullptr, r);
+    float c3[3], gq[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        c3[c] = rgb[3 * ray + c];
+        gq[c] = (c3[c] - rgb_gt[3 * ray + c]) * norm;
     }
+    float accum = fmaf(c3[0], gq[0], fmaf(c3[1], gq[1], c3[2] * gq[2]));
+    if (beta_per_ray > 0.f) {
+        const float tin = __expf(log_t_fwd[ray]);
+        accum += beta_per_ray * (1.f - tin / (1.f - tin + 1e-3f));
+    }
+    BwdRay<B> st(rc, lane, gq, accum, sparsity, &sh, go);
+    march_backward<DT, B, (WAVES <= 3)>(g, o, r, rc, lane, st, go, log, ray);
 }
 
 // Counting sort of the rays by descending cost in two launches: a histogram,
@@ -3725,9 +3712,8 @@ extern "C" int svox2_volume_render_cuvol_fused(const svox2_grid_t* grid,
                                dim3(blocks_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s, g,
                                dirs, rgb_gt, rgb_out, lt, beta, sparsity_loss, norm, go, rs);
             hipLaunchKernelGGL((k_render_backward_mse<DT, B, SVOX2_BWD_WAVES_FEW, true>),
-                               dim3(blocks_for(n_rays, kBlock)), dim3(kBlock), 0, s, g, o,
-                               origins, dirs, ray_clip, n_rays, rgb_gt, rgb_out, lt, beta,
-                               sparsity_loss, norm, static_cast<const uint32_t*>(nullptr), go,
+                               dim3(blocks), dim3(kBlock), 0, s, g, o, origins, dirs, ray_clip,
+                               n_rays, rgb_gt, rgb_out, lt, beta, sparsity_loss, norm, order, go,
                                rs, log);
             return;
         }
