@@ -812,8 +812,7 @@ def main():
                               "WRITE_SIZE of `bench.py --pmc`, calibrated on a 1 GiB copy)",
             "kernel": "fused call (float32 storage, SH-2): forward ray order "
                       "(k_ray_length_key, k_cost_hist, k_cost_scatter), k_render_rays_rec "
-                      "(recording the samples), k_rec_colours, backward ray order "
-                      "(k_cost_hist, k_cost_scatter), k_render_backward_replay, "
+                      "(recording the samples), k_rec_colours, k_render_backward_replay, "
                       "k_render_backward_mse (rays whose records overflowed)",
             "kernel_ms": head["kernel_ms"],
             "alg_bytes_per_launch": head["alg_bytes_per_launch"],
