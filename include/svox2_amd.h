@@ -69,8 +69,9 @@ typedef struct svox2_grid {
     int64_t sh_stride;      /* elements between SH rows (0 = sh_data_dim) */
     /* Optional (NULL = none) cell map of these links and rows, as written by
      * svox2_build_cell_map; it must be rebuilt whenever links or rows change.
-     * The march then decides skips and empty cells from it and reads the
-     * links only for cells with an occupied corner.  Results are the same. */
+     * The march then decides skips and empty cells from it, sampling decides
+     * empty cells, and both read the links only for cells with an occupied
+     * corner.  Results are the same. */
     const uint16_t* cell_map;
     /* Optional MSI background (NULL background_links = none), the
      * background_links / background_data of SparseGridSpec

@@ -250,8 +250,8 @@ class SparseGridSpec:
         self.basis_type: int = BASIS_TYPE_SH
         self.basis_data: Optional[torch.Tensor] = None
         # Cell map of the links (svox2_build_cell_map).  None: built on first
-        # use and cached per links tensor (rebuilt when the links change);
-        # False: the march reads links only.
+        # use and cached per links tensor (rebuilt when the links change), for
+        # the renderers alone; False: the march reads links only.
         self.cell_map = None
 
 
@@ -389,8 +389,8 @@ def _vec3(v) -> Tuple[float, float, float]:
 
 
 def _grid_struct(g: SparseGridSpec, need_sh: bool = True, need_map: bool = True,
-                 build_map: bool = True) -> _Grid:
-    """build_map False: use the links' cell map only if there is one already."""
+                 own_map: bool = False) -> _Grid:
+    """own_map: no cell map but the one the spec carries."""
     links = _check(g.links, "links", (torch.int32,), 3)
     dens = _check_rows(g.density_data, "density_data", _DATA_DTYPES)
     sh = g.sh_data
@@ -423,8 +423,8 @@ def _grid_struct(g: SparseGridSpec, need_sh: bool = True, need_map: bool = True,
     s.sh_stride = _row_stride(sh) if sh is not None else 0
     cmap = g.cell_map if need_map else False
     if cmap is None:
-        cmap = _cached_cell_map(links, dens.size(0), build_map)
-    if cmap is not False and cmap is not None:
+        cmap = False if own_map else _cached_cell_map(links, dens.size(0))
+    if cmap is not False:
         need = load_library().svox2_cell_map_bytes(s.size)
         _check(cmap, "cell_map", (torch.int16,), 1)
         if cmap.numel() * 2 < need or cmap.device != links.device:
@@ -462,8 +462,7 @@ _CELL_MAP_CACHE = 4
 _ACCEL_EPOCH: dict = {}
 
 
-def _cached_cell_map(links: torch.Tensor, rows: int, build: bool = True
-                     ) -> Optional[torch.Tensor]:
+def _cached_cell_map(links: torch.Tensor, rows: int) -> torch.Tensor:
     key = (links.device.index, links.data_ptr(), tuple(links.shape), links._version, int(rows),
            _ACCEL_EPOCH.get((links.device.index, links.data_ptr()), 0))
     stream = torch.cuda.current_stream(links.device)
@@ -477,8 +476,6 @@ def _cached_cell_map(links: torch.Tensor, rows: int, build: bool = True
             stream.wait_event(built)
             cmap.record_stream(stream)
         return cmap
-    if not build:
-        return None
     cmap = build_cell_map(links, rows)
     built = torch.cuda.Event()
     if not torch.cuda.is_current_stream_capturing():
@@ -857,21 +854,17 @@ def volume_render_nvol_fused(grid: SparseGridSpec, rays: RaysSpec, opt: RenderOp
               float(sparsity_loss), _ptr(rgb_out), ctypes.byref(gs), _stream(o))
 
 
-def _sample_struct(grid: SparseGridSpec, points: torch.Tensor, need_sh: bool) -> _Grid:
-    """The grid for sampling these points.  From 32768 points on it carries the
-    links' cell map if an earlier call built one, from 524288 on in any case
-    (building it takes 0.37 ms at 512^3 and saves 0.15 ms per million points and
-    pass); fewer points do not make up for the lookup."""
-    n = points.size(0)
-    return _grid_struct(grid, need_sh=need_sh, need_map=n >= 1 << 15,
-                        build_map=n >= 1 << 19 and not torch.cuda.is_current_stream_capturing())
-
-
 def sample_grid(grid: SparseGridSpec, points: torch.Tensor,
                 want_colors: bool) -> Tuple[torch.Tensor, torch.Tensor]:
-    """sample_grid (svox2_kernel.cu:181-217): (density (n,1), sh (n,C) or (0,C))."""
+    """sample_grid (svox2_kernel.cu:181-217): (density (n,1), sh (n,C) or (0,C)).
+
+    Sampling reads the spec's own tensors: links written without a change of
+    their version (through ``.data`` or by another library), made under
+    inference mode, or changed between two replays of a captured call are sampled
+    as they are.  So it takes a cell map only where the spec carries one (a million
+    points at 512^3, forward and backward: 0.32 ms without, 0.20 ms with it)."""
+    g = _grid_struct(grid, need_sh=bool(want_colors), own_map=True)
     _check(points, "points", (torch.float32,), 2)
-    g = _sample_struct(grid, points, bool(want_colors))
     if points.size(1) != 3:
         raise RuntimeError("points must be (n, 3)")
     n = points.size(0)
@@ -889,8 +882,8 @@ def sample_grid_backward(grid: SparseGridSpec, points: torch.Tensor,
                          grad_density_out: torch.Tensor, grad_sh_out: torch.Tensor,
                          want_colors: bool) -> None:
     """sample_grid_backward (svox2_kernel.cu:219-267)."""
+    g = _grid_struct(grid, need_sh=False, own_map=True)
     _check(points, "points", (torch.float32,), 2)
-    g = _sample_struct(grid, points, False)
     n = points.size(0)
     _check(grad_out_density, "grad_out_density", (torch.float32,), 2)
     _check_rows(grad_density_out, "grad_density_out", (torch.float32,), 1)

@@ -1,0 +1,106 @@
+"""Which calls take a cell map, and whose: sampling only the one its spec
+carries, so that it follows links however they were written; the renderers one
+that is cached per links tensor, built before it is read on every stream."""
+import pytest
+import torch
+
+from svox2_amd import _C, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(dev, reso=64, seed=7):
+    gen = torch.Generator().manual_seed(seed)
+    sc = scenes.make_blob_grid(reso, scenes.BlobSpec(4, (0.1, 0.1), (20.0, 20.0)), gen)
+    grid = scenes.to_sparse_grid(sc, device=dev)
+    grid.opt.sigma_thresh, grid.opt.stop_thresh = 1e-8, 1e-7
+    return grid
+
+
+def _rays(dev, n=2000, seed=3):
+    import svox2_amd
+    o, d = scenes.sphere_rays(n, torch.Generator().manual_seed(seed), radius=1.8, target=0.6)
+    return svox2_amd.Rays(o.to(dev), d.to(dev))
+
+
+def _fill_empty(links, rows):
+    """Gives every empty cell some row, through .data: the version stays."""
+    version = links._version
+    some = torch.arange(links.numel(), dtype=torch.int32, device=links.device) % rows
+    links.data.copy_(torch.where(links < 0, some.view(links.shape), links))
+    assert links._version == version
+
+
+@pytest.mark.parametrize("n", [40000, 600000])
+def test_sample_follows_links_without_a_version(gpu, n):
+    """Links changed through .data after a render: samples (and their adjoint)
+    are those of the links as they are, the same bits as without any map."""
+    grid = _grid(gpu)
+    with torch.no_grad():
+        grid.volume_render(_rays(gpu))
+    pts = torch.rand(n, 3, generator=torch.Generator().manual_seed(n)).to(gpu) * 2 - 1
+    _C.sample_grid(grid._to_cpp(), pts, True)
+    _fill_empty(grid.links, grid.sh_data.size(0))
+    bare = grid._to_cpp()
+    bare.cell_map = False
+    got, want = _C.sample_grid(grid._to_cpp(), pts, True), _C.sample_grid(bare, pts, True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    grid.sample(pts)[0].sum().backward()
+    weight = grid.density_data.grad.double().sum().item()
+    # Every point lies among cells with rows: its 8 weights sum to 1.
+    assert abs(weight - n) <= 1e-4 * n
+
+
+def test_sample_inference_links(gpu):
+    """Links made under inference mode have no version; they are sampled as any."""
+    grid = _grid(gpu)
+    pts = torch.rand(40000, 3, generator=torch.Generator().manual_seed(1)).to(gpu) * 2 - 1
+    spec = grid._to_cpp()
+    want = _C.sample_grid(spec, pts, True)
+    with torch.inference_mode():
+        spec.links = grid.links.clone()
+    assert all(torch.equal(a, b) for a, b in zip(_C.sample_grid(spec, pts, True), want))
+
+
+def test_captured_sample_follows_links(gpu):
+    """A captured sample reads the links at each replay, whatever became of the
+    renderers' cached maps in between."""
+    grid = _grid(gpu)
+    rays = _rays(gpu)
+    pts = torch.rand(1 << 19, 3, generator=torch.Generator().manual_seed(2)).to(gpu) * 2 - 1
+    spec, bare = grid._to_cpp(), grid._to_cpp()
+    bare.cell_map = False
+    with torch.no_grad():
+        grid.volume_render(rays)
+    _C.sample_grid(spec, pts, True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = _C.sample_grid(spec, pts, True)
+    for step in range(4):
+        graph.replay()
+        want = _C.sample_grid(bare, pts, True)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, want)), step
+        if step == 0:
+            grid.links[grid.links < 0] = 0
+        elif step == 1:
+            grid.accelerate()
+        else:
+            for seed in range(20 + 5 * step, 25 + 5 * step):  # drops the cached maps
+                with torch.no_grad():
+                    _grid(gpu, seed=seed).volume_render(rays)
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 65, 1000, 40001])
+def test_sample_own_map(gpu, n):
+    """A spec's own map is used whatever the point count, also where the last
+    wavefront's 16 points are not full: the same bits as without."""
+    grid = _grid(gpu)
+    pts = torch.rand(n, 3, generator=torch.Generator().manual_seed(n)).to(gpu) * 2.2 - 1.1
+    spec = grid._to_cpp()
+    out = []
+    for cmap in (False, _C.build_cell_map(spec.links, grid.sh_data.size(0))):
+        spec.cell_map = cmap
+        assert bool(_C._grid_struct(spec, own_map=True).cell_map) == (cmap is not False)
+        out.append(_C.sample_grid(spec, pts, True) + _C.sample_grid(spec, pts, False)[:1])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
