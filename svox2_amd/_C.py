@@ -251,7 +251,8 @@ class SparseGridSpec:
         self.basis_data: Optional[torch.Tensor] = None
         # Cell map of the links (svox2_build_cell_map).  None: built on first
         # use and cached per links tensor (rebuilt when the links change), for
-        # the renderers alone; False: the march reads links only.
+        # the renderers alone and not while a graph is captured; False: the
+        # march reads links only.
         self.cell_map = None
 
 
@@ -422,9 +423,9 @@ def _grid_struct(g: SparseGridSpec, need_sh: bool = True, need_map: bool = True,
     s.density_stride = _row_stride(dens)
     s.sh_stride = _row_stride(sh) if sh is not None else 0
     cmap = g.cell_map if need_map else False
-    if cmap is None:
-        cmap = False if own_map else _cached_cell_map(links, dens.size(0))
-    if cmap is not False:
+    if cmap is None and not own_map:
+        cmap = _cached_cell_map(links, dens.size(0))
+    if cmap is not None and cmap is not False:
         need = load_library().svox2_cell_map_bytes(s.size)
         _check(cmap, "cell_map", (torch.int16,), 1)
         if cmap.numel() * 2 < need or cmap.device != links.device:
@@ -462,7 +463,23 @@ _CELL_MAP_CACHE = 4
 _ACCEL_EPOCH: dict = {}
 
 
-def _cached_cell_map(links: torch.Tensor, rows: int) -> torch.Tensor:
+def _capturing(t: torch.Tensor) -> bool:
+    """Whether the current stream of the tensor's device is being captured."""
+    with _on_device(t):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _cached_cell_map(links: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
+    """The links' cell map, built on first use; None while a graph is captured.
+
+    A captured call reads the links alone: a map built by it would be written at
+    the replays only, and one from the cache has an owner who may drop it, while
+    the graph keeps its address and may be replayed after the links have changed.
+    A program that wants a map in a captured call keeps one itself, in the spec
+    (512^3, 800x800 image: 1.45 ms without, 0.99 ms with it; 65536 rays forward and
+    backward 0.72 and 0.67 ms, 5000 rays the same)."""
+    if _capturing(links):
+        return None
     key = (links.device.index, links.data_ptr(), tuple(links.shape), links._version, int(rows),
            _ACCEL_EPOCH.get((links.device.index, links.data_ptr()), 0))
     stream = torch.cuda.current_stream(links.device)
@@ -470,7 +487,7 @@ def _cached_cell_map(links: torch.Tensor, rows: int) -> torch.Tensor:
     if found is not None and not found[3].expired():
         _CELL_MAPS.move_to_end(key)
         cmap, built_on, built, _ = found
-        if stream != built_on and not torch.cuda.is_current_stream_capturing():
+        if stream != built_on:
             # Another stream's map: wait for its build, and keep its memory
             # until this stream's work is done.
             stream.wait_event(built)
@@ -478,8 +495,7 @@ def _cached_cell_map(links: torch.Tensor, rows: int) -> torch.Tensor:
         return cmap
     cmap = build_cell_map(links, rows)
     built = torch.cuda.Event()
-    if not torch.cuda.is_current_stream_capturing():
-        built.record(stream)
+    built.record(stream)
     # Drop stale maps of the same links tensor, then the oldest ones.
     for k in [k for k in _CELL_MAPS if k[:3] == key[:3]]:
         del _CELL_MAPS[k]

@@ -104,3 +104,38 @@ def test_sample_own_map(gpu, n):
         assert bool(_C._grid_struct(spec, own_map=True).cell_map) == (cmap is not False)
         out.append(_C.sample_grid(spec, pts, True) + _C.sample_grid(spec, pts, False)[:1])
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_captured_render(gpu, warm):
+    """A render captured before or after an eager one: an eager render between
+    the capture and the first replay, and every replay, have the bits of a render
+    without a map, also when the cached maps are dropped or the links change in
+    between."""
+    grid = _grid(gpu)
+    rays = _rays(gpu)
+    bare = grid._to_cpp()
+    bare.cell_map = False
+
+    def plain():
+        return _C.volume_render_cuvol(bare, rays._to_cpp(), grid.opt._to_cpp())
+
+    with torch.no_grad():
+        _grid(gpu, seed=9).volume_render(rays)  # kernels loaded
+        if warm:
+            grid.volume_render(rays)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = grid.volume_render(rays)
+        assert torch.equal(grid.volume_render(rays), plain())
+        for step in range(4):
+            graph.replay()
+            want = plain()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), step
+            if step == 0:
+                for seed in range(30, 36):  # drops the cached map
+                    _grid(gpu, seed=seed).volume_render(rays)
+            elif step == 1:
+                _fill_empty(grid.links, grid.sh_data.size(0))
+                assert not torch.equal(plain(), want)
