@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 from collections import OrderedDict
 from typing import Optional, Tuple
 
@@ -460,6 +461,7 @@ def _grid_struct(g: SparseGridSpec, need_sh: bool = True, need_map: bool = True,
 # pointer and so do not bump the tensor version.
 _CELL_MAPS: "OrderedDict[tuple, tuple]" = OrderedDict()
 _CELL_MAP_CACHE = 4
+_CELL_MAP_LOCK = threading.Lock()  # a look-up moves its entry, a build drops others
 _ACCEL_EPOCH: dict = {}
 
 
@@ -483,26 +485,27 @@ def _cached_cell_map(links: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
     key = (links.device.index, links.data_ptr(), tuple(links.shape), links._version, int(rows),
            _ACCEL_EPOCH.get((links.device.index, links.data_ptr()), 0))
     stream = torch.cuda.current_stream(links.device)
-    found = _CELL_MAPS.get(key)
-    if found is not None and not found[3].expired():
-        _CELL_MAPS.move_to_end(key)
-        cmap, built_on, built, _ = found
-        if stream != built_on:
-            # Another stream's map: wait for its build, and keep its memory
-            # until this stream's work is done.
-            stream.wait_event(built)
-            cmap.record_stream(stream)
+    with _CELL_MAP_LOCK:
+        found = _CELL_MAPS.get(key)
+        if found is not None and not found[3].expired():
+            _CELL_MAPS.move_to_end(key)
+            cmap, built_on, built, _ = found
+            if stream != built_on:
+                # Another stream's map: wait for its build, and keep its memory
+                # until this stream's work is done.
+                stream.wait_event(built)
+                cmap.record_stream(stream)
+            return cmap
+        cmap = build_cell_map(links, rows)
+        built = torch.cuda.Event()
+        built.record(stream)
+        # Drop stale maps of the same links tensor, then the oldest ones.
+        for k in [k for k in _CELL_MAPS if k[:3] == key[:3]]:
+            del _CELL_MAPS[k]
+        _CELL_MAPS[key] = (cmap, stream, built, StorageWeakRef(links.untyped_storage()))
+        while len(_CELL_MAPS) > _CELL_MAP_CACHE:
+            _CELL_MAPS.popitem(last=False)
         return cmap
-    cmap = build_cell_map(links, rows)
-    built = torch.cuda.Event()
-    built.record(stream)
-    # Drop stale maps of the same links tensor, then the oldest ones.
-    for k in [k for k in _CELL_MAPS if k[:3] == key[:3]]:
-        del _CELL_MAPS[k]
-    _CELL_MAPS[key] = (cmap, stream, built, StorageWeakRef(links.untyped_storage()))
-    while len(_CELL_MAPS) > _CELL_MAP_CACHE:
-        _CELL_MAPS.popitem(last=False)
-    return cmap
 
 
 def build_cell_map(links: torch.Tensor, rows: int) -> torch.Tensor:

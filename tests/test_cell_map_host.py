@@ -1,5 +1,7 @@
 """The renderers' cell map cache, its streams and events replaced by host objects."""
 import contextlib
+import threading
+from collections import OrderedDict
 
 import pytest
 import torch
@@ -43,7 +45,7 @@ def cache(monkeypatch):
         state.built.append(FakeMap(state.stream))
         return state.built[-1]
 
-    monkeypatch.setattr(_C, "_CELL_MAPS", type(_C._CELL_MAPS)())
+    monkeypatch.setattr(_C, "_CELL_MAPS", OrderedDict())
     monkeypatch.setattr(_C, "_ACCEL_EPOCH", {})
     monkeypatch.setattr(_C, "build_cell_map", build)
     monkeypatch.setattr(_C, "_on_device", lambda t: contextlib.nullcontext())
@@ -68,3 +70,24 @@ def test_capture_leaves_the_cache_alone(cache):
     assert _C._cached_cell_map(links, 3) is cmap and len(cache.built) == 1
     cache.capturing = True
     assert _C._cached_cell_map(links, 3) is None and len(_C._CELL_MAPS) == 1
+
+
+def test_two_threads(cache, monkeypatch):
+    """A thread that fills the cache while another looks a map up does not take
+    the found entry away under it."""
+    links = [_links(k) for k in range(6)]
+    fill = threading.Thread(target=lambda: [_C._cached_cell_map(x, 3) for x in links[1:]])
+
+    class Interrupted(OrderedDict):
+        def get(self, *args):
+            found = super().get(*args)
+            if found is not None and fill.ident is None:
+                fill.start()
+                fill.join(0.3)  # waits for as long as the other thread is kept out
+            return found
+
+    monkeypatch.setattr(_C, "_CELL_MAPS", Interrupted())
+    cmap = _C._cached_cell_map(links[0], 3)
+    assert _C._cached_cell_map(links[0], 3) is cmap
+    fill.join()
+    assert len(cache.built) == 6 and len(_C._CELL_MAPS) == _C._CELL_MAP_CACHE
