@@ -467,6 +467,8 @@ _ACCEL_EPOCH: dict = {}
 
 def _capturing(t: torch.Tensor) -> bool:
     """Whether the current stream of the tensor's device is being captured."""
+    if t.device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
     with _on_device(t):
         return torch.cuda.is_current_stream_capturing()
 
