@@ -49,6 +49,7 @@ def cache(monkeypatch):
     monkeypatch.setattr(_C, "_ACCEL_EPOCH", {})
     monkeypatch.setattr(_C, "build_cell_map", build)
     monkeypatch.setattr(_C, "_on_device", lambda t: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state.capturing)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: state.stream)
     monkeypatch.setattr(torch.cuda, "Event", FakeEvent)
@@ -91,3 +92,16 @@ def test_two_threads(cache, monkeypatch):
     assert _C._cached_cell_map(links[0], 3) is cmap
     fill.join()
     assert len(cache.built) == 6 and len(_C._CELL_MAPS) == _C._CELL_MAP_CACHE
+
+
+def test_streams_share_a_map(cache):
+    """A map is built once; every other stream waits for its build and keeps its
+    memory until that stream's work is done."""
+    links = _links()
+    a, b = FakeStream("a"), FakeStream("b")
+    cache.stream = a
+    cmap = _C._cached_cell_map(links, 3)
+    assert _C._cached_cell_map(links, 3) is cmap and not a.waited and not cmap.used_by
+    cache.stream = b
+    assert _C._cached_cell_map(links, 3) is cmap and len(cache.built) == 1
+    assert [e.recorded for e in b.waited] == [a] and cmap.used_by == [b]

@@ -139,3 +139,42 @@ def test_captured_render(gpu, warm):
             elif step == 1:
                 _fill_empty(grid.links, grid.sh_data.size(0))
                 assert not torch.equal(plain(), want)
+
+
+def test_render_on_several_streams(gpu):
+    """Renders on streams that take turns without waiting for each other, each
+    new grid's map wanted on all of them: the bits of a render without a map."""
+    rays = _rays(gpu)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    grids = [_grid(gpu, seed=40 + k) for k in range(3)]
+    out = []
+    torch.cuda.synchronize()
+    with torch.no_grad():
+        for k in range(9):
+            for grid in grids:
+                with torch.cuda.stream(streams[k % 3]):
+                    out.append((grid, grid.volume_render(rays)))
+    torch.cuda.synchronize()
+    for grid, got in out:
+        bare = grid._to_cpp()
+        bare.cell_map = False
+        assert torch.equal(got, _C.volume_render_cuvol(bare, rays._to_cpp(), grid.opt._to_cpp()))
+
+
+def test_map_ends_with_its_storage(gpu):
+    """Two links tensors that take turns at one address (both are views of the
+    same memory, each with a storage of its own) get a map each."""
+    grid = _grid(gpu)
+    rays = _rays(gpu)
+    memory = grid.links.clone()
+    spec = grid._to_cpp()
+    for flip in (False, True):
+        memory.copy_(grid.links.flip(0) if flip else grid.links)
+        spec.links = torch.from_dlpack(memory)
+        assert spec.links.data_ptr() == memory.data_ptr() and spec.links._version == 0
+        out = []
+        for cmap in (None, False):
+            spec.cell_map = cmap
+            out.append(_C.volume_render_cuvol(spec, rays._to_cpp(), grid.opt._to_cpp()))
+        assert torch.equal(out[0], out[1])
+        spec.links = None
