@@ -222,3 +222,28 @@ def test_load_legacy_data_layout(tmp_path):
     g.save(path2)
     z = np.load(path2)
     assert np.array_equal(z["background_links"], bl) and np.array_equal(z["background_data"], bd)
+
+
+@pytest.mark.parametrize("rays_per_launch", [7, 12, 24, 1000])
+def test_depth_image_launches(monkeypatch, rays_per_launch):
+    """A depth image is cut into launches of a bounded number of rays, the pixels
+    in order, whatever the batch size says."""
+    from svox2_amd import svox2 as facade
+    seen = []
+
+    def depth(self, rays, sigma_thresh=None):
+        assert sigma_thresh == 0.5
+        seen.append(rays.origins.size(0))
+        return rays.dirs[:, 0] + 10 * rays.dirs[:, 1]
+
+    monkeypatch.setattr(facade, "DEPTH_LAUNCH_RAYS", rays_per_launch)
+    monkeypatch.setattr(svox2_amd.SparseGrid, "volume_render_depth", depth)
+    grid = svox2_amd.SparseGrid(reso=8)
+    cam = svox2_amd.Camera(torch.eye(4), fx=20.0, width=6, height=4)
+    out = grid.volume_render_depth_image(cam, 0.5, batch_size=5)
+    dirs = cam.gen_rays().dirs
+    assert torch.equal(out, (dirs[:, 0] + 10 * dirs[:, 1]).view(4, 6))
+    assert sum(seen) == 24 and max(seen) <= rays_per_launch
+    # A launch has 32 threads a ray and must stay below 2^32 threads.
+    monkeypatch.undo()
+    assert facade.DEPTH_LAUNCH_RAYS * 32 < 2 ** 32
