@@ -326,6 +326,14 @@ size_t svox2_ray_order_workspace_bytes(int64_t n_rays);
  * counterpart in the reference. */
 size_t svox2_volume_render_cuvol_fused_workspace_bytes(int64_t n_rays);
 
+/* The same for one grid: more where the batch is recorded and at least a
+ * quarter of the cells have rows (up to 32 KiB per ray and 256 MiB, so that the
+ * records of longer rays fit), svox2_background_workspace_bytes with a
+ * background, which keeps neither records nor log.  No counterpart in the
+ * reference. */
+size_t svox2_volume_render_cuvol_fused_best_workspace_bytes(const svox2_grid_t* grid,
+                                                            int64_t n_rays);
+
 /* Device workspace bytes svox2_volume_render_cuvol_backward and
  * svox2_volume_render_cuvol_fused need for an n_rays batch over a grid with
  * a background: the ray-ordering workspace, then 16 bytes per ray (the

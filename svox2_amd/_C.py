@@ -49,6 +49,7 @@ EXPORTED_SYMBOLS = (
     "svox2_volume_render_cuvol_backward", "svox2_volume_render_cuvol_fused",
     "svox2_volume_render_cuvol_fused_noalloc",
     "svox2_ray_order_workspace_bytes", "svox2_volume_render_cuvol_fused_workspace_bytes",
+    "svox2_volume_render_cuvol_fused_best_workspace_bytes",
     "svox2_background_workspace_bytes", "svox2_cell_map_bytes",
     "svox2_build_cell_map", "svox2_volume_render_cuvol_tiles",
     "svox2_volume_render_cuvol_stats", "svox2_volume_render_expected_term",
@@ -210,6 +211,8 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     lib.svox2_cell_map_bytes.restype = ctypes.c_size_t
     lib.svox2_volume_render_cuvol_fused_workspace_bytes.argtypes = [i64]
     lib.svox2_volume_render_cuvol_fused_workspace_bytes.restype = ctypes.c_size_t
+    lib.svox2_volume_render_cuvol_fused_best_workspace_bytes.argtypes = [G, i64]
+    lib.svox2_volume_render_cuvol_fused_best_workspace_bytes.restype = ctypes.c_size_t
     lib.svox2_ray_order_workspace_bytes.argtypes = [i64]
     lib.svox2_ray_order_workspace_bytes.restype = ctypes.c_size_t
     lib.svox2_background_workspace_bytes.argtypes = [i64]
@@ -754,15 +757,8 @@ def volume_render_cuvol_fused(grid: SparseGridSpec, rays: RaysSpec, opt: RenderO
     # stream (from torch's caching allocator).
     lib = load_library()
     if ordered and record:
-        nbytes = lib.svox2_volume_render_cuvol_fused_workspace_bytes(o.size(0))
-        # More bytes hold more records: where most cells have rows, so that
-        # most samples contribute, rays outgrow the least, are marched twice and
-        # marched again by the backward (4096 rays of a dense 64^3 grid: 0.44 ms
-        # a step, 0.30 ms with room for all).  Up to 32 KiB per ray while that
-        # stays below 256 MiB.  Sparse grids keep to the least: their records fit,
-        # and spread over more memory they take 2 % longer.
-        if 4 * g.rows >= g.size[0] * g.size[1] * g.size[2]:
-            nbytes = max(nbytes, min(o.size(0) << 15, 256 << 20))
+        nbytes = lib.svox2_volume_render_cuvol_fused_best_workspace_bytes(ctypes.byref(g),
+                                                                          o.size(0))
     elif ordered:
         nbytes = lib.svox2_ray_order_workspace_bytes(o.size(0))
     else:
