@@ -838,17 +838,15 @@ __device__ __forceinline__ void write_log(const ChunkLog& log, const float* stag
     }
 }
 
-// Record stream of the fused call: the forward appends, per ray, a header and
-// one 96-byte record per contributing sample of each chunk; the backward
-// replays them instead of re-marching.  Slot s is rec[6 s .. 6 s + 5]
-// (float4).  Ray r owns slots [r * fixed, (r + 1) * fixed) and continues in
-// overflow blocks of kRecBlock slots taken with one atomic add.  Headers:
-// (n > 0, -) n records follow; (0, next) continue at slot next; (-1, -) end.
-// state[r] = 1 when the ray's stream is complete, 2 when the overflow region
-// ran out (the backward then re-marches the ray).
-//
-// The recorded chunks of all rays are listed in clist; the backward replays each
-// by itself.
+// Record stream of the fused call: the forward writes, per ray, for each chunk
+// with contributing samples a header (their count) and one 96-byte record per
+// sample; the backward replays them instead of re-marching.  Slot s is rec[6 s ..
+// 6 s + 5] (float4).  Ray r owns slots [r * fixed, (r + 1) * fixed) and continues
+// in overflow blocks of kRecBlock slots taken with one atomic add.  The recorded
+// chunks of all rays are listed in clist by their header's slot; the colours and
+// the backward take each by itself.  state[r] = 1 when all of the ray's chunks are
+// recorded and listed, 2 when a region ran out (the backward then re-marches the
+// ray).
 struct RecStream {
     float4* __restrict__ rec;
     int32_t* __restrict__ state;
@@ -869,7 +867,7 @@ struct RecStream {
     float4* __restrict__ ray_info;      // per ray: (first entry, entries, background term)
     int64_t clist_cap;
 };
-constexpr int kRecBlock = 64;  // >= 32 records + header + the end/jump header
+constexpr int kRecBlock = 64;  // >= 32 records + header
 constexpr int kRecParts = 64;  // counter partitions at most
 constexpr int kDeferChunks = 64;  // recorded chunks a ray can list for deferred colours
 constexpr int64_t kDeferCap = 9;  // chunk list entries per ray of the batch
@@ -885,15 +883,14 @@ __device__ __forceinline__ const float4* rec_field0(const float4* rec, int64_t s
     return rec + 6 * slot + 6;
 }
 
-__device__ __forceinline__ void put_header(float4* rec, int64_t slot, int n, int64_t next) {
-    rec[6 * slot] = make_float4(__int_as_float(n), __int_as_float(static_cast<int>(next)), 0.f,
-                                0.f);
+__device__ __forceinline__ void put_header(float4* rec, int64_t slot, int n) {
+    rec[6 * slot] = make_float4(__int_as_float(n), 0.f, 0.f, 0.f);
 }
 
 // Forward march of one ray.  out[3] = composited colour (all lanes),
 // returns the final log transmittance.  A chunk's colour sums its live
-// samples' weighted colours (per run group, then across the group); the ray's
-// colour is the sum of its chunks' in march order plus the background.
+// samples' weighted colours (chunk_colours); the ray's colour is the sum of its
+// chunks' in march order plus the background.
 //
 // DEFER (recording forward): the chunks' colours are left to k_rec_colours.
 // The samples are recorded with zero colours, each recorded chunk's header
@@ -968,8 +965,8 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                         for (int a = 0; a < 3; ++a) total[a] += sum[a];
                     }
                     if (RECORD && rec_ok) {
-                        // Header + n_live records; keep one slot for a jump/end header.
-                        if (cur + n_live + 2 > end) {
+                        // Header + n_live records.
+                        if (cur + n_live + 1 > end) {
                             const int part = static_cast<int>(ray % rs->parts);
                             uint32_t nb = 0;
                             if (lane == 0)
@@ -983,7 +980,6 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                                 const int64_t nxt = rs->overflow_base +
                                                     static_cast<int64_t>(nb) * rs->parts +
                                                     part * kRecBlock;
-                                if (lane == 0) put_header(rs->rec, cur, 0, nxt);
                                 cur = nxt;
                                 end = nxt + kRecBlock;
                             }
@@ -992,11 +988,11 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
                         if (rec_ok) {
                             const int k = n_rec_chunks++;
                             if (DEFER && defer && lane == 0) slot_lds[k] = static_cast<int32_t>(cur);
-                            if (lane == 0) put_header(rs->rec, cur, n_live, 0);
+                            if (lane == 0) put_header(rs->rec, cur, n_live);
                             if (c.live) {
                                 const int rank = __popc(c.live_mask & ((1u << lane) - 1u));
                                 float4* q = rec_field0(rs->rec, cur) + rank;
-                                q[0] = make_float4(c.p[0], c.p[1], c.p[2], __int_as_float(c.base));
+                                q[0] = make_float4(c.p[0], c.p[1], c.p[2], 0.f);
                                 q[n_live] = make_float4(__int_as_float(c.l[0]), __int_as_float(c.l[1]),
                                                         __int_as_float(c.l[2]), c.weight);
                                 q[2 * n_live] = make_float4(__int_as_float(c.lk[0]), __int_as_float(c.lk[1]),
@@ -1061,12 +1057,7 @@ __device__ __forceinline__ float march_forward(const GridView<DT>& g, const OptV
 #pragma unroll
     for (int a = 0; a < 3; ++a) out[a] = total[a] + tb;
     if (cost != nullptr) *cost = backward_cost(n_chunks);
-    if (RECORD) {
-        if (lane == 0) {
-            if (rec_ok) put_header(rs->rec, cur, -1, 0);
-            rs->state[ray] = rec_ok ? 1 : 2;
-        }
-    }
+    if (RECORD && lane == 0) rs->state[ray] = rec_ok ? 1 : 2;
     if (LOG) {
         const int n_logged = static_cast<int>(min(n_chunks, static_cast<uint32_t>(kLogChunks)));
         const int staged = n_logged % kLogStage;
@@ -2789,7 +2780,7 @@ inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
 size_t fused_workspace_bytes(int64_t n) {
     const int64_t order = static_cast<int64_t>(order_workspace_bytes(n));
     const int64_t state = align256(4 * n);
-    const int64_t counter = align256(4 * 4 * kRecParts);
+    const int64_t counter = align256(4 * 2 * kRecParts);
     const int64_t info = align256(16 * n);
     const int64_t clist = align256(8 * kDeferCap * n);
     const int64_t crgb = align256(16 * kDeferCap * n);
@@ -2816,7 +2807,7 @@ int64_t record_scale(size_t bytes, int64_t n) {
     const int64_t least = static_cast<int64_t>(fused_workspace_bytes(n));
     const int64_t per_ray = 24 * kDeferCap + kRecOverflow * kRecSlotBytes;
     const int64_t extra = static_cast<int64_t>(bytes) - least - 4 * 256;  // alignment
-    // Header slots are int32: at most 2^31 - 1 slots.
+    // Header slots are staged as int32: at most 2^31 - 1 slots.
     const int64_t most = 64 * (INT32_MAX - n * kRecFixed) / (n * kRecOverflow);
     return std::max<int64_t>(64, std::min<int64_t>(64 + 64 * extra / (n * per_ray), most));
 }
@@ -2836,7 +2827,7 @@ RecStream record_stream(void* ws, size_t bytes, int64_t n) {
     rs.state = reinterpret_cast<int32_t*>(p);
     p += align256(4 * n);
     rs.next_block = reinterpret_cast<uint32_t*>(p);
-    p += align256(4 * 4 * kRecParts);
+    p += align256(4 * 2 * kRecParts);
     rs.ray_info = reinterpret_cast<float4*>(p);
     p += align256(16 * n);
     rs.clist = reinterpret_cast<uint2*>(p);
@@ -3597,7 +3588,7 @@ extern "C" size_t svox2_ray_order_workspace_bytes(int64_t n_rays) {
 // MI355X: 0.780 against 0.855 ms at 65536 rays, 1.41 against 1.20 ms at
 // 131072, where the records' traffic outweighs the re-march).  Larger
 // batches re-march from the chunk log.  Slot indices must stay below 2^31
-// (headers hold them as int32).
+// (they are staged as int32).
 bool fused_records(int64_t n) {
     return (SVOX2_RECORD_ALL || n <= 2 * order_min_rays()) &&
            n * (kRecFixed + kRecOverflow) < INT32_MAX;
