@@ -352,14 +352,14 @@ __device__ __forceinline__ void bg_lds_fence() {
 // with dL/drgb is the running `accum` the reference carries over from the
 // grid's backward.
 //
-// The atomic requests bound this kernel (about 20 G/s, whatever their width):
-// added sample by sample, 4 requests of 32 bytes per live sample (34M for 65536
-// rays through 64 layers), it took 1.87 ms.  A ray turns by a fraction of a
-// pixel and crosses half a layer per sample, so consecutive samples share most
-// of their grid points: kept in registers until the ray leaves a grid point,
-// 1.36 ms; until it leaves a column or its 8 layers, so that a request carries
-// a column's 128 bytes, 1.25 ms (of
-// which 0.37 ms places and reads the samples and 0.21 ms are mask stores).
+// The atomic requests bound this kernel (about 20 G/s, whatever their width up to
+// 64 bytes): added sample by sample, 4 requests of 32 bytes per live sample (34M
+// for 65536 rays through 64 layers), it took 1.87 ms.  A ray turns by a fraction
+// of a pixel and crosses half a layer per sample, so consecutive samples share
+// most of their grid points: kept in registers until the ray leaves a grid point,
+// 1.36 ms; until it leaves a column or its 8 layers, so that one instruction adds
+// a column's 128 bytes (two requests), 1.25 ms (of which 0.37 ms places and reads
+// the samples and 0.10 ms are mask stores: 1.13 ms without a mask).
 __global__ __launch_bounds__(kBgBlock) void k_background_backward(
         BgView b, const float* __restrict__ origins, const float* __restrict__ dirs, int64_t n,
         const float* __restrict__ grad_in, const float* __restrict__ color_cache,
