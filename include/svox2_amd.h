@@ -290,12 +290,12 @@ int svox2_volume_render_cuvol_backward(const svox2_grid_t* grid,
  *   segment length in the grid, records each ray's chunk count, and the
  *   backward processes the rays in descending order of that count;
  * - at least svox2_volume_render_cuvol_fused_workspace_bytes(n_rays) bytes:
- *   for batches below that threshold the forward writes every contributing
+ *   for batches up to twice that threshold the forward writes every contributing
  *   sample (position, corner links, colour, transmittance) to a record
  *   stream in the workspace and the backward replays it instead of
  *   re-marching the ray (a ray whose records do not fit is re-marched; any
  *   bytes beyond hold more records);
- *   for batches at or above it the forward also logs where it placed the
+ *   for larger batches the forward logs where it placed the
  *   samples of each ray's first 16 chunks, and the backward evaluates those
  *   chunks from the log instead of placing them again.
  * A grid with a background needs a workspace of at least
